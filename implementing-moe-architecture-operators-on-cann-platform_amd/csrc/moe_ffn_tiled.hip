@@ -6,18 +6,29 @@
 // With ~1000 rows per expert (T = 8192, K = 2, E = 16) the GEMMs have an arithmetic intensity of ~1500 flop/B
 // against HBM, far above the MFMA ridge. Both are "NT": activation rows and weight rows are contiguous along the
 // reduction dim k.
-//   macro tile   256 activation rows x 256 weight rows x 64 k per stage; 8 waves (2 x 4), each a 128 x 64
-//                sub-tile (8 x 4 v_mfma_f32_16x16x32_f16 tiles, 128 fp32 accumulators per lane). The weight
-//                fragment is the MFMA's first operand, so each lane ends with 4 consecutive output columns of one
-//                row and the epilogue stores 8 bytes at a time.
+//   macro tile   256 activation rows x 256 weight rows x 64 k per stage; 8 waves (2 x 4), each 128 x 64 as four
+//                quadrants of 64 rows x 32 weight rows (4 x 2 v_mfma_f32_16x16x32_f16 tiles, 128 fp32 accumulators
+//                per lane in all). The weight fragment is the MFMA's first operand, so each lane ends with 4
+//                consecutive output columns of one row.
 //   copies       each stage is copied from global memory straight into LDS (buffer_load ... lds: no staging
 //                registers, no LDS store instructions; 32-bit offsets against buffer resources whose range ends
 //                at the buffer, so a read past it returns zeros instead of faulting)
-//   ring         two LDS slots. Stage q's 64 MFMAs per wave run in four phases of 16; the LDS fragment reads a
-//                later phase needs are issued between the MFMAs of the phase before (sched_group_barrier), so
-//                both pipes stay busy. One barrier per stage, between the third and the fourth phase: by then
-//                the wave has read all of stage q, and stage q + 1 has landed, so the barrier publishes q + 1
-//                and frees q's slot for the copies of q + 2.
+//   ticks        a stage is four pairs of ticks, one pair per quadrant: a memory tick (LDS reads of the quadrant's
+//                new fragments, 2 copy instructions) and a compute tick (16 MFMAs), a barrier after each. Waves 4-7
+//                run one tick behind waves 0-3, and wave w shares its SIMD with wave w + 4, so on every SIMD one
+//                wave's MFMAs run beside the other's reads and copies.
+//   ring         two LDS slots of four 16 KB half tiles (two of activation rows, two of weight rows). A half tile is
+//                free one tick pair after its last read and is refilled at once, so the copies leave evenly over the
+//                stage, 2 per wave and tick pair, 7 tick pairs ahead of their use; the waits are counted
+//                (vmcnt(12): all but the youngest 6 half tiles). With the 8 copies of a stage issued together after
+//                one barrier per stage (64 KB in a quarter of its MFMA time) the waves stalled on issuing them:
+//                prefill (T = 8192, H = 2048, E = 16, K = 2, I = 8192) gate/up 1024 -> 939 us, down 506 -> 447 us;
+//                Mixtral (T = 4096, H = 4096, E = 8, I = 14336) 1743 -> 1644 us, 878 -> 791 us; T = 3001, H = 1056,
+//                E = 24, K = 3, I = 736 64 -> 56 us.
+//                What bounds it now is power: on all-zero inputs prefill gate/up takes 721 us (942 us before), on
+//                random ones the clock falls to 1.62 GHz with the MFMAs busy 72 % of it. 32x32x16 MFMAs are 9 %
+//                slower for that reason, and MFMAs sharing the weight instead of the activation fragment 1 %;
+//                s_setprio around the compute tick changes nothing.
 //   persistent   one workgroup per CU walks its tiles back to back and the ring runs on across them: the
 //                copies of a tile's first two stages go out during the previous tile's last two. The tile table
 //                (per-expert tile prefix and row offsets) is built once per workgroup in LDS, so finding a tile
@@ -30,15 +41,16 @@
 //                allocation at tile changes.
 //   LDS layout   unpadded 128-byte rows of 8 granules of 16 B; granule g of row r is stored at g ^ ((r >> 1) & 7),
 //                so the 16 rows one ds_read_b128 touches (same logical granule) spread over all banks
-//   gate/up      the 256 weight rows of a tile are, per wave quarter, 32 W_gate rows and the matching 32 W_up
-//                rows, so each wave holds gate and up of the same (row, i) and applies SwiGLU in registers
-//                (hardware exp2 and reciprocal, ~1 ulp each), writing fp16 hidden rows
+//   gate/up      weight half 0 of a tile is 128 W_gate rows, half 1 the matching W_up rows, so each wave holds gate
+//                and up of the same (row, i) and applies SwiGLU in registers (hardware exp2 and reciprocal, ~1 ulp
+//                each), writing fp16 hidden rows
 //   down         weight rows are W_down rows (output columns); the epilogue writes expert_out[slot] directly
 //   scheduling   tiles are (expert, n-tile, m-tile) with m fastest. Workgroups are dispatched round-robin over
 //                the 8 XCDs; each XCD owns a contiguous range of tiles, so the m-tiles that share a weight tile
 //                share that XCD's L2.
-// Rows past an expert's count are clamped to its last row on load and masked on store. A reduction extent that is
-// an odd multiple of 32 ends with a half stage (KT instantiation): its upper 32 columns are cleared in LDS.
+// Rows past an expert's count repeat its last row (gate/up) or read zeros (down) and are masked on store. A reduction
+// extent that is an odd multiple of 32 ends with a half stage (KT instantiation): only its first 32-k step is
+// multiplied.
 
 #include "moe_device.h"
 #include "moe_launch.h"
@@ -53,6 +65,7 @@ constexpr int kBK = 64;            // k per stage
 constexpr int kPitch = kBK;        // LDS row pitch in halfs (granules XOR-swizzled)
 constexpr int kThreads = 512;      // 8 waves
 constexpr int kStageHalfs = (kBM + kBN) * kPitch;
+constexpr int kHalfTile = 128 * kPitch;  // halfs of one of a stage's four half tiles
 constexpr int kNStage = 2;
 constexpr int kLdsBytes = kNStage * kStageHalfs * 2;  // the ring; the tile table follows it
 constexpr int kEpiStageBytes = kThreads / kWave * 2048;  // down epilogue: 16 rows x 128 B per wave
@@ -107,9 +120,9 @@ __device__ __forceinline__ XcdSched xcd_sched(int x, int total, int nloc, int ns
     return s;
 }
 
-// Barrier of the copy ring. The only LDS writes of the main loop are this wave's direct-to-LDS copies, which the
-// caller's explicit vmcnt wait covers, and every fragment read of the stage has fed an MFMA before the wave gets
-// here. A workgroup-scope release fence would also wait for the copies still in flight (vmcnt(0)).
+// Barrier between two ticks. The only LDS writes of the main loop are the direct-to-LDS copies, which the memory
+// ticks' explicit vmcnt waits cover, and the memory ticks also wait for their LDS reads. A workgroup-scope release
+// fence would wait for the copies still in flight too (vmcnt(0)).
 __device__ __forceinline__ void ring_barrier() {
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
@@ -128,9 +141,7 @@ __device__ __forceinline__ float swiglu_fast(float g, float u) {
 // once and keeps them live across the main loop, where the accumulators and fragments leave no room for them:
 // they are spilled, and each reload in the tile change or the epilogue waits (vmcnt) for every stage copy in
 // flight. A volatile read cannot be hoisted, so what make_plan and the epilogue derive from it is recomputed there.
-// Used by the down projection (spills 44 -> 28 and 24 -> 12 registers; on one box DeepSeek-V2-Lite down
-// 606-608 -> 568-571 us, prefill 496-499 -> 488-491 us, Mixtral 874 -> 868-869 us). Gate/up keeps lane_id(): its
-// code is unchanged, and with the fresh index it ran 0.5-1 % slower.
+// Used by the down projection.
 __device__ __forceinline__ int lane_fresh() {
     int v;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(v));
@@ -139,18 +150,6 @@ __device__ __forceinline__ int lane_fresh() {
 
 enum Epilogue { kSwiGLU = 0, kScatter = 1 };
 
-// Interleave pattern of one 16-MFMA phase: NR LDS reads and NV global->LDS copies are issued one after each of
-// its first MFMAs, so neither pipe waits for the other.
-template <int NR, int NV>
-__device__ __forceinline__ void phase_sched() {
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-        if (q < NR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
-        if (q < NV) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // VMEM read
-    }
-}
-
 // One work item: tile (e, mt, nt), k-stages [k0, k0 + nk), and the partial slot it writes (-1: the whole k
 // range, written through the epilogue).
 struct TileRef {
@@ -158,18 +157,20 @@ struct TileRef {
     int k0, nk, part;
 };
 
-// Copy plan of one tile: per stage and operand, wave w issues 4 instructions j, each filling 8 whole LDS rows
-// r = (4 w + j) * 8 + lane / 8 (128 B each); lane fetches global granule (lane % 8) ^ ((r >> 1) & 7). ao / bo
-// are byte offsets of those granules at k = 0 in the activation and weight buffers ar / wr.
+// Copy plan of one tile. A stage is four half tiles of 128 rows x 128 B (activation rows 0-127 and 128-255, and the
+// two weight halves); per half tile wave w issues 2 instructions j, each filling 8 whole LDS rows
+// r = (2 w + j) * 8 + lane / 8; lane fetches global granule (lane % 8) ^ ((r >> 1) & 7). ao / bo are byte offsets of
+// those granules at k = 0 in the activation and weight buffers ar / wr; the second weight half lies bhalf bytes
+// after the first (and, for hidden rows, the second activation half ahalf bytes after the first).
 struct CopyPlan {
-    uint32_t ao[4], bo[4];
+    uint32_t ao[4], bo[2];
     __amdgpu_buffer_rsrc_t ar, wr;
 };
 
 // SPLIT: the leftover round may be split over k (p.split); a separate instantiation, so the kernel without it
 // keeps its register allocation at tile changes. KT: the reduction extent is an odd multiple of 32, so the last
-// k-stage holds 32 valid columns; its copies read on into the next row (or past the buffer, as zeros), and the
-// waves zero those granules in LDS before the stage is published.
+// k-stage holds 32 valid columns; its copies read on into the next row (or past the buffer, as zeros), and those
+// columns are not multiplied.
 template <int EPI, bool SPLIT, bool KT = false>
 __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
     extern __shared__ __align__(16) uint16_t lds[];
@@ -285,22 +286,24 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
         }
     };
     auto make_plan = [&](const TileRef& T, int buf, CopyPlan& P) __attribute__((always_inline)) {
+        const int ln = EPI == kScatter ? lane_fresh() : lane;  // lane_fresh: see above
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            // the down projection reads the lane index afresh (lane_fresh)
-            const int r = (wave * 4 + j) * 8 + ((EPI == kScatter ? lane_fresh() : lane) / 8);
-            const uint32_t gq = static_cast<uint32_t>(((EPI == kScatter ? lane_fresh() : lane) % 8) ^ ((r >> 1) & 7));
-            if (p.gather) {
-                P.ao[j] = static_cast<uint32_t>(rowtab[buf * kBM + r] / p.K) * kbytes + gq * 16;
-            } else {  // rows relative to the tile's first row
-                P.ao[j] = static_cast<uint32_t>(min(r, T.ne - 1 - T.mt * kBM)) * kbytes + gq * 16;
+        for (int j = 0; j < 2; ++j) {
+            const int r = (wave * 2 + j) * 8 + ln / 8;
+            const uint32_t gq = static_cast<uint32_t>((ln % 8) ^ ((r >> 1) & 7));
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (p.gather) {  // rows past the tile's last repeat it
+                    P.ao[h * 2 + j] = static_cast<uint32_t>(rowtab[buf * kBM + h * 128 + r] / p.K) * kbytes + gq * 16;
+                } else {  // rows relative to the tile's first row; those past its last are past the buffer: zeros
+                    P.ao[h * 2 + j] = static_cast<uint32_t>(h * 128 + r) * kbytes + gq * 16;
+                }
             }
-            if (EPI == kSwiGLU) {
-                const int quarter = r >> 6, sub = r & 63;
-                const int ic = min(T.nt * 128 + quarter * 32 + (sub & 31), p.I - 1);
-                P.bo[j] = ((sub < 32 ? 0u : static_cast<uint32_t>(p.I)) + static_cast<uint32_t>(ic)) * static_cast<uint32_t>(p.H) * 2 + gq * 16;
-            } else {
-                const int n = min(T.nt * kBN + r, p.H - 1);
+            if (EPI == kSwiGLU) {  // half 0: W_gate rows, half 1: the matching W_up rows
+                const int ic = min(T.nt * 128 + r, p.I - 1);
+                P.bo[j] = static_cast<uint32_t>(ic) * static_cast<uint32_t>(p.H) * 2 + gq * 16;
+            } else {  // half h of wave column wn: output columns wn * 64 + h * 32 + [0, 32); past H: past the buffer
+                const int n = T.nt * kBN + (r >> 5) * 64 + (r & 31);
                 P.bo[j] = (2u * static_cast<uint32_t>(p.I) * p.H + static_cast<uint32_t>(n) * p.I) * 2 + gq * 16;
             }
         }
@@ -317,165 +320,85 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
                                                  static_cast<int>(3u * static_cast<uint32_t>(p.I) * p.H * 2), 0x00020000);
     };
 
-    // copies stage kc of plan P into ring slot q % 2. The data is consumed from LDS, so the loads bypass the L1
-    // (sc0); they still allocate in L2, where the other m-tiles of the weight tile find them (a non-temporal hint
-    // there made the kernel 35 % slower).
-    auto copy = [&](int q, int kc, const CopyPlan& P) __attribute__((always_inline)) {
-        const int kb = kc * kBK * 2;  // byte offset of the stage along k (scalar)
-        uint16_t* sa = lds + (q % kNStage) * kStageHalfs;
-        uint16_t* sb = sa + kBM * kPitch;
+    // copies one half tile of stage kc of plan P into ring slot q % 2. The data is consumed from LDS, so the loads
+    // bypass the L1 (sc0); they still allocate in L2, where the other m-tiles of the weight tile find them (a
+    // non-temporal hint there made the kernel 35 % slower).
+    const int bhalf = EPI == kSwiGLU ? p.I * p.H * 2 : 32 * p.I * 2;  // bytes from weight half 0 to half 1
+    auto copyA = [&](int q, int h, int kc, const CopyPlan& P) __attribute__((always_inline)) {
+        uint16_t* s = lds + (q % kNStage) * kStageHalfs + h * kHalfTile;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(P.ar, (__attribute__((address_space(3))) void*)(sa + (wave * 4 + j) * 8 * kPitch), 16,
-                                                     static_cast<int>(P.ao[j]), kb, 0, kCopyPolicy);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(P.wr, (__attribute__((address_space(3))) void*)(sb + (wave * 4 + j) * 8 * kPitch), 16,
-                                                     static_cast<int>(P.bo[j]), kb, 0, kCopyPolicy);
-        }
+        for (int j = 0; j < 2; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(P.ar, (__attribute__((address_space(3))) void*)(s + (wave * 2 + j) * 8 * kPitch), 16,
+                                                     static_cast<int>(P.ao[h * 2 + j]), kc * kBK * 2, 0, kCopyPolicy);
     };
-    f32x4 acc[8][4];
-    // Fragment registers: the wave's 128 rows are two halves of 4 16-row blocks (A0, A1); the 64 weight rows are
-    // 4 blocks, held for the even (Bx) and the odd (By) 32-k step of a stage.
-    f16x8 A0[4], A1[4], Bx[4], By[4];
+    auto copyB = [&](int q, int h, int kc, const CopyPlan& P) __attribute__((always_inline)) {
+        uint16_t* s = lds + (q % kNStage) * kStageHalfs + (2 + h) * kHalfTile;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(P.wr, (__attribute__((address_space(3))) void*)(s + (wave * 2 + j) * 8 * kPitch), 16,
+                                                     static_cast<int>(P.bo[j]), kc * kBK * 2 + h * bhalf, 0, kCopyPolicy);
+    };
+    // acc[hA][hB]: 4 x 2 blocks of 16 x 16. Fragments: one activation half (4 blocks, both 32-k steps) and both
+    // weight halves (2 blocks each).
+    f32x4 acc[2][2][4][2];
+    f16x8 fa[2][4], fb0[2][2], fb1[2][2];
     const int sw = (row16 >> 1) & 7;
-    auto rdA = [&](int q, int kk, int h, f16x8 (&a)[4]) __attribute__((always_inline)) {
-        const uint16_t* sa = lds + (q % kNStage) * kStageHalfs + (wm * 128 + h * 64 + row16) * kPitch + (((kk * 4 + kg) ^ sw) * 8);
+    auto rdA = [&](int q, int h) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = *reinterpret_cast<const f16x8*>(sa + i * 16 * kPitch);
-    };
-    auto rdB = [&](int q, int kk, f16x8 (&bb)[4]) __attribute__((always_inline)) {
-        const uint16_t* sb = lds + (q % kNStage) * kStageHalfs + (kBM + wn * 64 + row16) * kPitch + (((kk * 4 + kg) ^ sw) * 8);
+        for (int kk = 0; kk < 2; ++kk) {
+            const uint16_t* s = lds + (q % kNStage) * kStageHalfs + h * kHalfTile + (wm * 64 + row16) * kPitch + (((kk * 4 + kg) ^ sw) * 8);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bb[j] = *reinterpret_cast<const f16x8*>(sb + j * 16 * kPitch);
-    };
-    // D[weight row][activation row]: each lane ends with 4 consecutive output columns of one row
-    auto mma = [&](int h, const f16x8 (&a)[4], const f16x8 (&bb)[4], bool zero) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                acc[h * 4 + i][j] = mfma16x16x32(bb[j], a[i], zero ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[h * 4 + i][j]);
-    };
-
-    // The ring of two LDS slots runs over this workgroup's tiles back to back: ring index q counts stages over
-    // all its tiles, and the copies of a tile's first two stages are issued during the previous tile's last two.
-    // Stage q multiplies its two 32-k steps in four phases of 16 MFMAs: (kk0, A0), (kk0, A1), (kk1, A0),
-    // (kk1, A1). Each phase reads the fragments that the next phase or the one after needs. Between the third and
-    // the fourth phase the wave has read all of stage q from LDS: one barrier then publishes stage q + 1 (every
-    // wave's copies have landed) and frees slot q % 2 for the copies of ring stage q + 2 (stage kc of plan P).
-    // After the last tile those copies repeat its last stage into the free slot and the fourth phase reads
-    // fragments nobody uses.
-    // KT: this wave's copy rows of ring stage qn, logical granules 4-7 (k 32-63 of the stage) set to zero; the lane
-    // that copied a granule clears it, after its own copies have landed (vmcnt) and before the barrier that
-    // publishes the stage (the caller's lgkmcnt(0) covers these writes)
-    auto zero_tail = [&](int qn) __attribute__((always_inline)) {
-        uint16_t* sa = lds + (qn % kNStage) * kStageHalfs;
-        uint16_t* sb = sa + kBM * kPitch;
-        const int ln = lane_fresh();
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int r = (wave * 4 + j) * 8 + ln / 8;
-            if (((ln % 8) ^ ((r >> 1) & 7)) >= 4) {
-                *reinterpret_cast<u32x4*>(sa + (wave * 4 + j) * 8 * kPitch + ln * 8) = u32x4{0u, 0u, 0u, 0u};
-                *reinterpret_cast<u32x4*>(sb + (wave * 4 + j) * 8 * kPitch + ln * 8) = u32x4{0u, 0u, 0u, 0u};
-            }
+            for (int i = 0; i < 4; ++i) fa[kk][i] = *reinterpret_cast<const f16x8*>(s + i * 16 * kPitch);
         }
     };
-    auto stage = [&](int q, bool first, int kc, const CopyPlan& P, bool tail_next) __attribute__((always_inline)) {
+    auto rdB = [&](int q, int h, f16x8 (&fb)[2][2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const uint16_t* s = lds + (q % kNStage) * kStageHalfs + (2 + h) * kHalfTile + (wn * 32 + row16) * kPitch + (((kk * 4 + kg) ^ sw) * 8);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) fb[kk][j] = *reinterpret_cast<const f16x8*>(s + j * 16 * kPitch);
+        }
+    };
+    // ends a memory tick: the fragments just read are in registers, and all but this wave's youngest 12 copies (6 half
+    // tiles) have landed, the half tile of the next memory tick among them; the barrier publishes it
+    auto tick_m = [&]() __attribute__((always_inline)) {
         __builtin_amdgcn_sched_barrier(0);
-        mma(0, A0, Bx, first);
-        rdA(q, 0, 1, A1);
-        rdB(q, 1, By);
-        phase_sched<8, 0>();
-        __builtin_amdgcn_sched_barrier(0);
-        mma(1, A1, Bx, first);
-        rdA(q, 1, 0, A0);
-        phase_sched<4, 0>();
-        __builtin_amdgcn_sched_barrier(0);
-        mma(0, A0, By, false);
-        rdA(q, 1, 1, A1);
-        phase_sched<4, 0>();
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // this wave's copies of ring stage q + 1
-        if (KT && tail_next) zero_tail(q + 1);
-        __builtin_amdgcn_s_waitcnt(0xc07f);        // lgkmcnt(0): this wave's reads of ring stage q are done
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(12) & 0xf0ffu);
         ring_barrier();
-        copy(q + 2, kc, P);
-        mma(1, A1, By, false);
-        rdB(q + 1, 0, Bx);
-        rdA(q + 1, 0, 0, A0);
-        phase_sched<8, 8>();
-        __builtin_amdgcn_sched_barrier(0);
     };
-
-    // Down projection: the same stage as a ring of 4 activation blocks of 16 rows, each read 3 blocks ahead of its
-    // MFMAs (16 blocks per stage, 8 per 32-k step, numbered on across stages so that block n sits in Ar[n % 4]),
-    // and the 4 weight blocks of each step (B0 even, B1 odd). 48 fragment registers instead of 64: the split
-    // kernel spills 24 registers instead of 57, and the down projection runs 0.5-3 % faster (prefill 508.6 ->
-    // 498-499 us, DeepSeek-V2-Lite 627 -> 607 us, Mixtral 892 -> 888 us; gate/up ran 1 % slower this way). The
-    // barrier comes before the odd step's seventh block, when the wave has read all of stage q; the last two
-    // blocks read stage q + 1's B0 and first 3 blocks.
-    f16x8 B0[4], B1[4], Ar[4];
-    auto rdA1 = [&](int q, int kk, int i) __attribute__((always_inline)) -> f16x8 {
-        return *reinterpret_cast<const f16x8*>(lds + (q % kNStage) * kStageHalfs + (wm * 128 + i * 16 + row16) * kPitch +
-                                               (((kk * 4 + kg) ^ sw) * 8));
+    // a compute tick: D[weight row][activation row], each lane ends with 4 consecutive output columns of one row
+    auto tick_c = [&](f32x4 (&c)[4][2], const f16x8 (&fb)[2][2], bool zero, bool half) __attribute__((always_inline)) {
+        auto mma = [&](int kk) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    c[i][j] = mfma16x16x32(fb[kk][j], fa[kk][i], zero && kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : c[i][j]);
+        };
+        mma(0);
+        if (!KT || !half) mma(1);
+        ring_barrier();
     };
-    auto rdB1 = [&](int q, int kk, int j) __attribute__((always_inline)) -> f16x8 {
-        return *reinterpret_cast<const f16x8*>(lds + (q % kNStage) * kStageHalfs + (kBM + wn * 64 + j * 16 + row16) * kPitch +
-                                               (((kk * 4 + kg) ^ sw) * 8));
-    };
-    auto stage_ring = [&](int q, bool first, int kc, const CopyPlan& P, bool tail_next) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            __builtin_amdgcn_sched_barrier(0);
-            Ar[(i + 3) % 4] = rdA1(q, (i + 3) / 8, (i + 3) % 8);
-            if (i < 4) B1[i] = rdB1(q, 1, i);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = mfma16x16x32(B0[j], Ar[i % 4], first ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[i][j]);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-                if (u < (i < 4 ? 2 : 1)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            __builtin_amdgcn_sched_barrier(0);
-            if (i < 5) Ar[(i + 3) % 4] = rdA1(q, 1, i + 3);
-            if (i == 6) {
-                __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // this wave's copies of ring stage q + 1
-                if (KT && tail_next) zero_tail(q + 1);
-                __builtin_amdgcn_s_waitcnt(0xc07f);        // lgkmcnt(0): this wave's reads of ring stage q are done
-                ring_barrier();
-                copy(q + 2, kc, P);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) B0[j] = rdB1(q + 1, 0, j);
-                Ar[0] = rdA1(q + 1, 0, 0);
-                Ar[1] = rdA1(q + 1, 0, 1);
-            }
-            if (i == 7) Ar[2] = rdA1(q + 1, 0, 2);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = mfma16x16x32(B1[j], Ar[(i + 8) % 4], acc[i][j]);
-            if (i == 6) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);  // 2 copies
-                    if (u < 3) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // 2 DS reads
-                }
-            } else {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-                    if (u == 0 && (i < 5 || i == 7)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
-                }
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    // tail_next: ring stage q + 1 is the last k-stage (KT)
-    auto run_stage = [&](int q, bool first, int kc, const CopyPlan& P, bool tail_next) __attribute__((always_inline)) {
-        if constexpr (EPI == kScatter) stage_ring(q, first, kc, P, tail_next);
-        else stage(q, first, kc, P, tail_next);
+    // One 64-k stage q: four memory ticks, each followed by a compute tick of 16 MFMAs (8 when `half`: the last
+    // stage of an odd multiple of 32). The copies are those of stage kc of plan P into the same slot, each half tile
+    // one tick pair after its last read.
+    auto stage = [&](int q, bool first, int kc, const CopyPlan& P, bool half) __attribute__((always_inline)) {
+        rdA(q, 0);
+        copyB(q, 0, kc, P);
+        tick_m();
+        tick_c(acc[0][0], fb0, first, half);
+        rdB(q, 1, fb1);
+        copyA(q, 0, kc, P);
+        tick_m();
+        tick_c(acc[0][1], fb1, first, half);
+        rdA(q, 1);
+        copyB(q, 1, kc, P);
+        tick_m();
+        tick_c(acc[1][0], fb0, first, half);
+        rdB(q + 1, 0, fb0);
+        copyA(q, 1, kc, P);
+        tick_m();
+        tick_c(acc[1][1], fb1, first, half);
     };
 
     CopyPlan plan;
@@ -483,19 +406,17 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     __syncthreads();
     make_plan(cur, 0, plan);
-    copy(0, SPLIT ? cur.k0 : 0, plan);
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // this wave's copies of stage 0 are in LDS
-    ring_barrier();                            // and every wave's
-    copy(1, SPLIT ? cur.k0 + 1 : 1, plan);
-    if constexpr (EPI == kScatter) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) B0[j] = rdB1(0, 0, j);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) Ar[i] = rdA1(0, 0, i);
-    } else {
-        rdB(0, 0, Bx);
-        rdA(0, 0, 0, A0);
+    for (int st = 0; st < 2; ++st) {
+        const int kc = (SPLIT ? cur.k0 : 0) + st;
+        copyB(st, 0, kc, plan);
+        copyA(st, 0, kc, plan);
+        copyB(st, 1, kc, plan);
+        copyA(st, 1, kc, plan);
     }
+    tick_m();  // the first half tiles of stage 0
+    rdB(0, 0, fb0);
+    tick_m();
     int q0 = 0;  // ring index of the current item's first stage
     for (int k = 0;; ++k) {
         TileRef nxt;
@@ -507,44 +428,51 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
         const int nk0 = SPLIT ? nxt.k0 : 0;
         const int kc0 = has_next ? nk0 : k0 + nk - 1, kc1 = has_next ? nk0 + 1 : k0 + nk - 1;
         const bool tail = KT && k0 + nk == nst;  // this item ends with the 32-column k-stage
-        if (nk > 2) {
-            run_stage(q0, true, k0 + 2, plan, false);
-            for (int s = 1; s + 2 < nk; ++s) run_stage(q0 + s, false, k0 + s + 2, plan, false);
-            if (has_next) make_plan(nxt, (k + 1) % 3, plan);
-            run_stage(q0 + nk - 2, false, kc0, plan, tail);
-            run_stage(q0 + nk - 1, false, kc1, plan, false);
-        } else {  // the next tile's plan is needed before the first barrier: wait for its row table here
+        if (nk < 4) {  // the next plan is needed before the counted waits cover its row table's copy: wait here
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
             __syncthreads();
-            if (has_next) make_plan(nxt, (k + 1) % 3, plan);
-            run_stage(q0, true, kc0, plan, tail);
-            run_stage(q0 + 1, false, kc1, plan, false);
         }
+        if (wm) ring_barrier();  // waves 4-7 run one tick behind waves 0-3
+        if (nk > 2) {
+            stage(q0, true, k0 + 2, plan, false);
+            for (int s = 1; s + 2 < nk; ++s) stage(q0 + s, false, k0 + s + 2, plan, false);
+            if (has_next) make_plan(nxt, (k + 1) % 3, plan);
+            stage(q0 + nk - 2, false, kc0, plan, false);
+        } else {
+            if (has_next) make_plan(nxt, (k + 1) % 3, plan);
+            stage(q0, true, kc0, plan, false);
+        }
+        stage(q0 + nk - 1, false, kc1, plan, tail);
+        if (!wm) ring_barrier();
 
-        // ---- epilogue: acc[i][j] lane holds D[weight row 4*kg + r of block j][activation row row16 of block i],
+        // ---- epilogue: a lane of acc[a][b][i][j] holds D[weight row 4*kg + r of block j of weight half b][activation row
+        // row16 of block i of activation half a],
         // i.e. 4 consecutive output columns of one row: one 8-byte store per (i, j) ----
-        const int m = cur.mt * kBM + wm * 128 + row16;
+        const int m = cur.mt * kBM + wm * 64 + row16;
         if (SPLIT && cur.part >= 0) {
             // a piece of a split tile: the raw fp32 sums of its k-range, [activation row][weight row] of the tile
             const int lane_e = lane_fresh(), row16 = lane_e & 15, kg = lane_e >> 4;
-            float* dst = p.partial + static_cast<size_t>(cur.part) * (kBM * kBN) + (wm * 128 + row16) * kBN + wn * 64 + kg * 4;
+            float* dst = p.partial + static_cast<size_t>(cur.part) * (kBM * kBN) + (wm * 64 + row16) * kBN + wn * 64 + kg * 4;
 #pragma unroll
             for (int i = 0; i < 8; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(dst + i * 16 * kBN + j * 16) = acc[i][j];
+                for (int j = 0; j < 4; ++j)
+                    *reinterpret_cast<f32x4*>(dst + ((i >> 2) * 128 + (i & 3) * 16) * kBN + j * 16) = acc[i >> 2][j >> 1][i & 3][j & 1];
         } else if (EPI == kSwiGLU) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                if (m + i * 16 >= cur.ne) continue;
-                uint16_t* dst = p.out + static_cast<size_t>(cur.off + m + i * 16) * p.I;
+                const int mi = m + (i >> 2) * 128 + (i & 3) * 16;
+                if (mi >= cur.ne) continue;
+                uint16_t* dst = p.out + static_cast<size_t>(cur.off + mi) * p.I;
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     const int col = cur.nt * 128 + wn * 32 + j * 16 + kg * 4;
                     if (col >= p.I) continue;
-                    const uint32_t lo = f32_to_f16_bits(swiglu_fast(acc[i][j][0], acc[i][j + 2][0])) |
-                                        (static_cast<uint32_t>(f32_to_f16_bits(swiglu_fast(acc[i][j][1], acc[i][j + 2][1]))) << 16);
-                    const uint32_t hi = f32_to_f16_bits(swiglu_fast(acc[i][j][2], acc[i][j + 2][2])) |
-                                        (static_cast<uint32_t>(f32_to_f16_bits(swiglu_fast(acc[i][j][3], acc[i][j + 2][3]))) << 16);
+                    const f32x4 g = acc[i >> 2][0][i & 3][j], u = acc[i >> 2][1][i & 3][j];
+                    const uint32_t lo = f32_to_f16_bits(swiglu_fast(g[0], u[0])) |
+                                        (static_cast<uint32_t>(f32_to_f16_bits(swiglu_fast(g[1], u[1]))) << 16);
+                    const uint32_t hi = f32_to_f16_bits(swiglu_fast(g[2], u[2])) |
+                                        (static_cast<uint32_t>(f32_to_f16_bits(swiglu_fast(g[3], u[3]))) << 16);
                     *reinterpret_cast<uint2*>(dst + col) = make_uint2(lo, hi);
                 }
             }
@@ -562,8 +490,9 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
             for (int i = 0; i < 8; ++i) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const uint32_t lo = f32_to_f16_bits(acc[i][j][0]) | (static_cast<uint32_t>(f32_to_f16_bits(acc[i][j][1])) << 16);
-                    const uint32_t hi = f32_to_f16_bits(acc[i][j][2]) | (static_cast<uint32_t>(f32_to_f16_bits(acc[i][j][3])) << 16);
+                    const f32x4 v = acc[i >> 2][j >> 1][i & 3][j & 1];
+                    const uint32_t lo = f32_to_f16_bits(v[0]) | (static_cast<uint32_t>(f32_to_f16_bits(v[1])) << 16);
+                    const uint32_t hi = f32_to_f16_bits(v[2]) | (static_cast<uint32_t>(f32_to_f16_bits(v[3])) << 16);
                     *reinterpret_cast<uint2*>(stg + row16 * 128 + (((2 * j + (kg >> 1)) ^ (row16 & 7)) << 4) + ((kg & 1) << 3)) =
                         make_uint2(lo, hi);
                 }
@@ -577,7 +506,7 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const int r = wm * 128 + i * 16 + h * 8 + rr;  // row of the tile
+                    const int r = (i >> 2) * 128 + wm * 64 + (i & 3) * 16 + h * 8 + rr;  // row of the tile
                     if (cur.mt * kBM + r >= cur.ne || col >= p.H) continue;
                     *reinterpret_cast<u32x4*>(p.out + static_cast<size_t>(rowtab[(k % 3) * kBM + r]) * p.H + col) = v[h];
                 }

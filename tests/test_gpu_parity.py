@@ -1410,3 +1410,22 @@ def test_decode_uses_streaming_and_prefill_uses_tiled():
     assert ffn_schedule(8192, 2048, 16, 2, 8192) == 1
     assert ffn_schedule(16384, 2048, 64, 6, 1408) == 1
     assert ffn_schedule(4096, 4096, 8, 2, 14336) == 1
+
+
+@pytest.mark.parametrize("H,I", [(96, 96), (128, 128), (160, 192), (192, 224), (256, 288), (320, 160), (416, 576)])
+def test_tiled_tile_and_stage_edges(ops, H, I):
+    """The tiled kernels at the edges of their 256 x 256 tiles (0 to 513 rows per expert, around 128 and 256; H and I
+    around 128 and 256 columns) and with reductions of 2 to 9 stages of 64, whole and ending in a half stage.
+    Bounds: expert_out is of order one (|values| < 8); the fp16 rounding of the I intermediates (2^-11 each, adding
+    in quadrature) and of the result (2^-11) stay below 8 * 2^-10 each in the worst element and 2^-10 in the mean."""
+    rows = [1, 127, 128, 129, 255, 256, 257, 64, 0, 385, 513, 192]
+    E, T = len(rows), sum(rows)
+    assert ffn_schedule(T, H, E, 1, I) == 1
+    rng = np.random.default_rng(H * 1000 + I)
+    ids = rng.permutation(np.repeat(np.arange(E, dtype=np.int32), rows)).reshape(T, 1)
+    x = rng.standard_normal((T, H), dtype=np.float32).astype(np.float16)
+    w = np.ones((T, 1), dtype=np.float16)
+    ew = np.concatenate([rng.standard_normal((E, 2 * I, H), dtype=np.float32) / math.sqrt(H),
+                         rng.standard_normal((E, I, H), dtype=np.float32) / math.sqrt(I)], axis=1).astype(np.float16)
+    eo = f32(host(ops.MoeExpertFFN(dev(x), dev(ids), dev(w), dev(ew))))
+    within(oracle.compare(eo, oracle_ffn_threads(f32(x), ids, f32(ew), I)), max_abs=2**-6, mean_abs=2**-10, cos=0.9999)
