@@ -6,33 +6,39 @@
 // With ~1000 rows per expert (T = 8192, K = 2, E = 16) the GEMMs have an arithmetic intensity of ~1500 flop/B
 // against HBM, far above the MFMA ridge. Both are "NT": activation rows and weight rows are contiguous along the
 // reduction dim k.
-//   macro tile   256 activation rows x 256 weight rows x 64 k per stage; 8 waves (2 x 4), each 128 x 64 as four
-//                quadrants of 64 rows x 32 weight rows (4 x 2 v_mfma_f32_16x16x32_f16 tiles, 128 fp32 accumulators
-//                per lane in all). The weight fragment is the MFMA's first operand, so each lane ends with 4
-//                consecutive output columns of one row.
+//   macro tile   256 activation rows x 256 weight rows x 64 k per stage; 8 waves (2 x 4), each 128 x 64 as two
+//                halves of 64 rows (4 x 4 v_mfma_f32_16x16x32_f16 tiles each, 128 fp32 accumulators per lane in
+//                all). The weight fragment is the MFMA's first operand, so each lane ends with 4 consecutive output
+//                columns of one row.
 //   copies       each stage is copied from global memory straight into LDS (buffer_load ... lds: no staging
 //                registers, no LDS store instructions; 32-bit offsets against buffer resources whose range ends
 //                at the buffer, so a read past it returns zeros instead of faulting)
-//   ticks        a stage is four pairs of ticks, one pair per quadrant: a memory tick (LDS reads of the quadrant's
-//                new fragments, 2 copy instructions) and a compute tick (16 MFMAs), a barrier after each. Waves 4-7
-//                run one tick behind waves 0-3, and wave w shares its SIMD with wave w + 4, so on every SIMD one
-//                wave's MFMAs run beside the other's reads and copies.
+//   ticks        a stage is two pairs of ticks, one pair per activation half: a memory tick (LDS reads of the
+//                half's fragments, copies) and a compute tick (32 MFMAs), a barrier after each. Waves 4-7 run one
+//                tick behind waves 0-3, and wave w shares its SIMD with wave w + 4, so on every SIMD one wave's
+//                MFMAs run beside the other's reads and copies.
 //   ring         two LDS slots of four 16 KB half tiles (two of activation rows, two of weight rows). A half tile is
-//                free one tick pair after its last read and is refilled at once, so the copies leave evenly over the
-//                stage, 2 per wave and tick pair, 7 tick pairs ahead of their use; the waits are counted
-//                (vmcnt(12): all but the youngest 6 half tiles). With the 8 copies of a stage issued together after
-//                one barrier per stage (64 KB in a quarter of its MFMA time) the waves stalled on issuing them:
-//                prefill (T = 8192, H = 2048, E = 16, K = 2, I = 8192) gate/up 1024 -> 939 us, down 506 -> 447 us;
-//                Mixtral (T = 4096, H = 4096, E = 8, I = 14336) 1743 -> 1644 us, 878 -> 791 us; T = 3001, H = 1056,
-//                E = 24, K = 3, I = 736 64 -> 56 us.
-//                What bounds it now is power: on all-zero inputs prefill gate/up takes 721 us (942 us before), on
-//                random ones the clock falls to 1.62 GHz with the MFMAs busy 72 % of it. 32x32x16 MFMAs are 9 %
-//                slower for that reason, and MFMAs sharing the weight instead of the activation fragment 1 %;
-//                s_setprio around the compute tick changes nothing.
+//                free one tick after its last read and is refilled at once, a whole stage ahead of its use, with
+//                counted waits (all but the youngest 8 copies of a wave). With the 8 copies a wave issues per stage
+//                sent together after the stage's one barrier (64 KB in a quarter of its MFMA time) the waves
+//                stalled on issuing them. Kernel times on one box each, that kernel -> this one (an in-between
+//                form with four tick pairs of 16 MFMAs a stage in the middle):
+//                  T = 8192, H = 2048, E = 16, K = 2, I = 8192: gate/up 1024 -> 917 -> 888 us, down 506 -> 440 -> 438
+//                  T = 16384, H = 2048, E = 64, K = 6, I = 1408: gate/up 1093 -> 965 -> 940 us, down 587 -> 515 -> 513
+//                What bounds it now is power: on all-zero inputs the first gate/up takes 700 us (942 us in the old
+//                kernel), on random ones the clock falls to ~1.6 GHz. On zeros, without any copies it would take
+//                ~120 us less (L2 misses: with every copy an L2 hit 613 instead of 728 us), without the epilogue
+//                ~60 us less, without the LDS reads nothing less (timing-only copies of the kernel). Measured and
+//                not kept: 32x32x16 MFMAs (9 % slower), MFMAs that share the weight instead of the activation
+//                fragment (1 % slower), copies issued between the MFMAs of the compute ticks (2-7 % slower, they
+//                leave later), the first k-stage rotated per XCD and other cache policies of the copies (level),
+//                s_setprio around the compute tick (level), skipping the second half's ticks in tiles of at most
+//                128 rows (1-3 % slower: such a tile takes as long, and the workgroups that share its weight tile
+//                drift apart).
 //   persistent   one workgroup per CU walks its tiles back to back and the ring runs on across them: the
 //                copies of a tile's first two stages go out during the previous tile's last two. The tile table
 //                (per-expert tile prefix and row offsets) is built once per workgroup in LDS, so finding a tile
-//                is a short LDS binary search; the next tile's 256 sorted-slot entries are copied into LDS a tile
+//                is a short search from the last tile's expert on; the next tile's 256 sorted-slot entries are copied into LDS a tile
 //                ahead.
 //   split        (down) the down projection has only ~2 tiles per CU at prefill, so a count-based schedule
 //                leaves the last round mostly idle: the tiles left over after the full rounds are split over k
@@ -43,12 +49,13 @@
 //                so the 16 rows one ds_read_b128 touches (same logical granule) spread over all banks
 //   gate/up      weight half 0 of a tile is 128 W_gate rows, half 1 the matching W_up rows, so each wave holds gate
 //                and up of the same (row, i) and applies SwiGLU in registers (hardware exp2 and reciprocal, ~1 ulp
-//                each), writing fp16 hidden rows
+//                each). Lanes exchange halves of their columns (v_permlane16_swap) and store 16 bytes each, 64 B a
+//                row (8-byte stores, 32 B a row: 905 instead of 892 us at prefill).
 //   down         weight rows are W_down rows (output columns); the epilogue writes expert_out[slot] directly
 //   scheduling   tiles are (expert, n-tile, m-tile) with m fastest. Workgroups are dispatched round-robin over
 //                the 8 XCDs; each XCD owns a contiguous range of tiles, so the m-tiles that share a weight tile
 //                share that XCD's L2.
-// Rows past an expert's count repeat its last row (gate/up) or read zeros (down) and are masked on store. A reduction
+// Rows past an expert's count read zeros (past the buffer) and are masked on store. A reduction
 // extent that is an odd multiple of 32 ends with a half stage (KT instantiation): only its first 32-k step is
 // multiplied.
 
@@ -146,6 +153,13 @@ __device__ __forceinline__ int lane_fresh() {
     int v;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(v));
     return v;
+}
+
+// Two fp32 values as packed fp16, each rounded to nearest even.
+__device__ __forceinline__ uint32_t pack_f16(float lo, float hi) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef f16 f16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, f16x2));
 }
 
 enum Epilogue { kSwiGLU = 0, kScatter = 1 };
@@ -251,22 +265,19 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
             }
             t = xs.base + loc;
         }
-        int lo = 0, hi = p.E;  // tab[lo] <= t < tab[hi]
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (__builtin_amdgcn_readfirstlane(tab[mid]) <= t) lo = mid;
-            else hi = mid;
-        }
+        int lo = T.e;  // the expert with tab[lo] <= t < tab[lo + 1], from the last tile's on
+        while (__builtin_amdgcn_readfirstlane(tab[lo + 1]) <= t) ++lo;
         T.e = lo;
         T.off = __builtin_amdgcn_readfirstlane(offs[lo]);
         T.ne = __builtin_amdgcn_readfirstlane(offs[lo + 1]) - T.off;
         const int mtiles = (T.ne + kBM - 1) / kBM;
         const int local = t - __builtin_amdgcn_readfirstlane(tab[lo]);
-        T.nt = local / mtiles;
+        T.nt = __builtin_amdgcn_readfirstlane(local / mtiles);  // the division runs on the VALU
         T.mt = local - T.nt * mtiles;
         return true;
     };
     TileRef cur;
+    cur.e = 0;
     if (!tile_at(0, cur)) return;
 
     // activation rows a tile copies: gate/up gathers token rows (x), down reads its own sorted hidden rows
@@ -286,16 +297,18 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
         }
     };
     auto make_plan = [&](const TileRef& T, int buf, CopyPlan& P) __attribute__((always_inline)) {
-        const int ln = EPI == kScatter ? lane_fresh() : lane;  // lane_fresh: see above
+        const int ln = lane_fresh();
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int r = (wave * 2 + j) * 8 + ln / 8;
             const uint32_t gq = static_cast<uint32_t>((ln % 8) ^ ((r >> 1) & 7));
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                if (p.gather) {  // rows past the tile's last repeat it
-                    P.ao[h * 2 + j] = static_cast<uint32_t>(rowtab[buf * kBM + h * 128 + r] / p.K) * kbytes + gq * 16;
-                } else {  // rows relative to the tile's first row; those past its last are past the buffer: zeros
+                // rows past the tile's last are past the buffer: zeros, and no memory traffic
+                if (p.gather) {
+                    const uint32_t row = static_cast<uint32_t>(rowtab[buf * kBM + h * 128 + r] / p.K);
+                    P.ao[h * 2 + j] = T.mt * kBM + h * 128 + r < T.ne ? row * kbytes + gq * 16 : 0x80000000u;
+                } else {  // rows relative to the tile's first row
                     P.ao[h * 2 + j] = static_cast<uint32_t>(h * 128 + r) * kbytes + gq * 16;
                 }
             }
@@ -338,9 +351,9 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(P.wr, (__attribute__((address_space(3))) void*)(s + (wave * 2 + j) * 8 * kPitch), 16,
                                                      static_cast<int>(P.bo[j]), kc * kBK * 2 + h * bhalf, 0, kCopyPolicy);
     };
-    // acc[hA][hB]: 4 x 2 blocks of 16 x 16. Fragments: one activation half (4 blocks, both 32-k steps) and both
-    // weight halves (2 blocks each).
-    f32x4 acc[2][2][4][2];
+    // Accumulators acc[hA][hB]: 4 x 2 blocks of 16 x 16. Fragments: one activation half (4 blocks, both 32-k steps)
+    // and both weight halves (2 blocks each).
+    using Acc = f32x4[2][4][2];
     f16x8 fa[2][4], fb0[2][2], fb1[2][2];
     const int sw = (row16 >> 1) & 7;
     auto rdA = [&](int q, int h) __attribute__((always_inline)) {
@@ -359,46 +372,132 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
             for (int j = 0; j < 2; ++j) fb[kk][j] = *reinterpret_cast<const f16x8*>(s + j * 16 * kPitch);
         }
     };
-    // ends a memory tick: the fragments just read are in registers, and all but this wave's youngest 12 copies (6 half
-    // tiles) have landed, the half tile of the next memory tick among them; the barrier publishes it
-    auto tick_m = [&]() __attribute__((always_inline)) {
+    // Ends a memory tick: the fragments just read are in registers, and all but this wave's youngest 8 copies have
+    // landed, the half tiles of the next memory tick among them; the barrier publishes them. `stores` (0, 8 or 16):
+    // at least that many stores of the last tile's epilogue are younger than the copies waited for and need not
+    // have ended.
+    auto tick_m = [&](int stores = 0) __attribute__((always_inline)) {
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(12) & 0xf0ffu);
+        if (stores == 8) __builtin_amdgcn_s_waitcnt(vmcnt_imm(16) & 0xf0ffu);
+        else if (stores == 16) __builtin_amdgcn_s_waitcnt(vmcnt_imm(24) & 0xf0ffu);
+        else __builtin_amdgcn_s_waitcnt(vmcnt_imm(8) & 0xf0ffu);
         ring_barrier();
     };
-    // a compute tick: D[weight row][activation row], each lane ends with 4 consecutive output columns of one row
-    auto tick_c = [&](f32x4 (&c)[4][2], const f16x8 (&fb)[2][2], bool zero, bool half) __attribute__((always_inline)) {
+    // A compute tick: D[weight row][activation row], each lane ends with 4 consecutive output columns of one row.
+    // half: the last stage of an odd multiple of 32, only its first 32-k step is multiplied.
+    auto tick_c = [&](Acc& c, bool zero, bool half) __attribute__((always_inline)) {
         auto mma = [&](int kk) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    c[i][j] = mfma16x16x32(fb[kk][j], fa[kk][i], zero && kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : c[i][j]);
+                for (int j = 0; j < 4; ++j)
+                    c[j >> 1][i][j & 1] = mfma16x16x32(j < 2 ? fb0[kk][j & 1] : fb1[kk][j & 1], fa[kk][i], zero && kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : c[j >> 1][i][j & 1]);
         };
         mma(0);
         if (!KT || !half) mma(1);
         ring_barrier();
     };
-    // One 64-k stage q: four memory ticks, each followed by a compute tick of 16 MFMAs (8 when `half`: the last
-    // stage of an odd multiple of 32). The copies are those of stage kc of plan P into the same slot, each half tile
-    // one tick pair after its last read.
-    auto stage = [&](int q, bool first, int kc, const CopyPlan& P, bool half) __attribute__((always_inline)) {
+    // The two tick pairs of 64-k stage q. half1 reads the first activation half and both weight halves, half2 the
+    // second activation half. Each refills what the memory tick before it read last: half1 the second activation
+    // half of stage q + 1 (stage kc of plan P), half2 the other three half tiles of stage q + 2 (again kc of P).
+    int stores = 0;  // stores of this wave's last epilogue, younger than the copies that stage 0 waits for
+    auto half1 = [&](Acc (&acc)[2], int q, bool first, int kc, const CopyPlan& P, bool half) __attribute__((always_inline)) {
         rdA(q, 0);
-        copyB(q, 0, kc, P);
-        tick_m();
-        tick_c(acc[0][0], fb0, first, half);
+        rdB(q, 0, fb0);
         rdB(q, 1, fb1);
-        copyA(q, 0, kc, P);
-        tick_m();
-        tick_c(acc[0][1], fb1, first, half);
+        copyA(q + 1, 1, kc, P);
+        tick_m(first ? stores : 0);
+        tick_c(acc[0], first, half);
+    };
+    auto half2 = [&](Acc (&acc)[2], int q, bool first, int kc, const CopyPlan& P, bool half) __attribute__((always_inline)) {
         rdA(q, 1);
+        copyA(q, 0, kc, P);
+        copyB(q, 0, kc, P);
         copyB(q, 1, kc, P);
-        tick_m();
-        tick_c(acc[1][0], fb0, first, half);
-        rdB(q + 1, 0, fb0);
-        copyA(q, 1, kc, P);
-        tick_m();
-        tick_c(acc[1][1], fb1, first, half);
+        tick_m(first ? stores : 0);
+        tick_c(acc[1], first, half);
+    };
+
+    // Epilogue: a lane of acc[a][b][i][j] holds D[weight row 4 * kg + r of block j of weight half b][activation row
+    // row16 of block i of activation half a], i.e. 4 consecutive output columns of one row.
+    auto epilogue = [&](const Acc (&acc)[2], const TileRef& cur, const int* rows) __attribute__((always_inline)) {
+        const int lane_e = lane_fresh(), row16 = lane_e & 15, kg = lane_e >> 4;
+        if (SPLIT && cur.part >= 0) {
+            // a piece of a split tile: the raw fp32 sums of its k-range, [activation row][weight row] of the tile
+            float* dst = p.partial + static_cast<size_t>(cur.part) * (kBM * kBN) + (wm * 64 + row16) * kBN + wn * 64 + kg * 4;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    *reinterpret_cast<f32x4*>(dst + ((i >> 2) * 128 + (i & 3) * 16) * kBN + j * 16) = acc[i >> 2][j >> 1][i & 3][j & 1];
+            }
+        } else if (EPI == kSwiGLU) {
+            // stored through a buffer that ends with the tile's rows; columns past I go past it too
+            const int row0 = cur.mt * kBM;
+            const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(p.out + static_cast<size_t>(cur.off + row0) * p.I, 0,
+                                                                                min(kBM, cur.ne - row0) * p.I * 2, 0x00020000);
+            const int col = cur.nt * 128 + wn * 32 + (kg & 1) * 16 + (kg >> 1) * 8;
+            const uint32_t at = col < p.I ? static_cast<uint32_t>((wm * 64 + row16) * p.I + col) * 2 : 0x80000000u;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                uint32_t v[2][2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const f32x4 g = acc[i >> 2][0][i & 3][j], u = acc[i >> 2][1][i & 3][j];
+                    // each value converted by itself: the last product and the rounding to fp16 are then one
+                    // v_fma_mixlo_f16, rounded once
+                    v[j][0] = f32_to_f16_bits(swiglu_fast(g[0], u[0])) |
+                              (static_cast<uint32_t>(f32_to_f16_bits(swiglu_fast(g[1], u[1]))) << 16);
+                    v[j][1] = f32_to_f16_bits(swiglu_fast(g[2], u[2])) |
+                              (static_cast<uint32_t>(f32_to_f16_bits(swiglu_fast(g[3], u[3]))) << 16);
+                }
+                // odd rows of 16 lanes of block 0 against even ones of block 1: each lane then holds 8 columns in a row
+                const auto lo = __builtin_amdgcn_permlane16_swap(v[0][0], v[1][0], false, false);
+                const auto hi = __builtin_amdgcn_permlane16_swap(v[0][1], v[1][1], false, false);
+                __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo[0], hi[0], lo[1], hi[1]}, hr, static_cast<int>(at), ((i >> 2) * 128 + (i & 3) * 16) * p.I * 2, 0);
+            }
+        } else {
+            // Whole-line stores: the wave's 128 x 64 sub-tile leaves as 16 instructions of 8 rows x 128 B. Row
+            // block i passes through the wave's own 2 KB of LDS (16 rows x 128 B; 16-byte granule g of row r at
+            // g ^ (r & 7)): lane (row16, kg) writes its four packed 4-column groups, then lane L reads granule
+            // L % 8 of row h * 8 + L / 8 (h = 0, 1). Stored straight from the MFMA layout (16 rows x 32 B per
+            // instruction) the epilogue cost ~100 us per DeepSeek-V2-Lite down launch (T = 16384, E = 64, K = 6).
+            uint8_t* stg = reinterpret_cast<uint8_t*>(lds) + tiled_epi_stage_offset(p.E) + wave * 2048;
+            // Rows past the tile's last and columns past H repeat the last valid row or granule, its data too: no
+            // divergent branch, and a full tile issues exactly 16 stores.
+            const int ncol = p.H - cur.nt * kBN - wn * 64;  // valid columns of the wave
+            if (ncol <= 0) return;
+            const int rr = lane_e >> 3, gq = min(lane_e & 7, (ncol - 1) >> 3);
+            const int col = cur.nt * kBN + wn * 64 + gq * 8;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int r0 = (i >> 2) * 128 + wm * 64 + (i & 3) * 16;  // the block's first row of the tile
+                const int last = min(15, cur.ne - cur.mt * kBM - r0 - 1);
+                if (last < 0) continue;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const f32x4 v = acc[i >> 2][j >> 1][i & 3][j & 1];
+                    *reinterpret_cast<uint2*>(stg + row16 * 128 + (((2 * j + (kg >> 1)) ^ (row16 & 7)) << 4) + ((kg & 1) << 3)) =
+                        make_uint2(pack_f16(v[0], v[1]), pack_f16(v[2], v[3]));
+                }
+                // the reads take what other lanes of this wave just wrote (LDS operations of one wave run in order)
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                u32x4 v[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int r = min(h * 8 + rr, last);
+                    v[h] = *reinterpret_cast<const u32x4*>(stg + r * 128 + ((gq ^ (r & 7)) << 4));
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // read before the next block's writes
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int r = r0 + min(h * 8 + rr, last);
+                    *reinterpret_cast<u32x4*>(p.out + static_cast<size_t>(rows[r]) * p.H + col) = v[h];
+                }
+            }
+        }
     };
 
     CopyPlan plan;
@@ -409,17 +508,15 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
         const int kc = (SPLIT ? cur.k0 : 0) + st;
-        copyB(st, 0, kc, plan);
         copyA(st, 0, kc, plan);
+        copyB(st, 0, kc, plan);
         copyB(st, 1, kc, plan);
-        copyA(st, 1, kc, plan);
+        if (st == 0) copyA(st, 1, kc, plan);
     }
     tick_m();  // the first half tiles of stage 0
-    rdB(0, 0, fb0);
-    tick_m();
     int q0 = 0;  // ring index of the current item's first stage
     for (int k = 0;; ++k) {
-        TileRef nxt;
+        TileRef nxt = cur;
         const bool has_next = tile_at(k + 1, nxt);
         // table k + 1 % 3 was last read two tiles ago; the barriers of tile k - 1 separate those reads from this copy
         if (has_next) load_rows(nxt, (k + 1) % 3);
@@ -433,85 +530,29 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
             __syncthreads();
         }
         if (wm) ring_barrier();  // waves 4-7 run one tick behind waves 0-3
+        Acc acc[2];
+        auto full = [&](int s, bool first) __attribute__((always_inline)) {
+            half1(acc, q0 + s, first, k0 + s + 1, plan, false);
+            half2(acc, q0 + s, first, k0 + s + 2, plan, false);
+        };
         if (nk > 2) {
-            stage(q0, true, k0 + 2, plan, false);
-            for (int s = 1; s + 2 < nk; ++s) stage(q0 + s, false, k0 + s + 2, plan, false);
+            full(0, true);
+            for (int s = 1; s + 2 < nk; ++s) full(s, false);
+            half1(acc, q0 + nk - 2, false, k0 + nk - 1, plan, false);
             if (has_next) make_plan(nxt, (k + 1) % 3, plan);
-            stage(q0 + nk - 2, false, kc0, plan, false);
+            half2(acc, q0 + nk - 2, false, kc0, plan, false);
         } else {
+            half1(acc, q0, true, k0 + 1, plan, false);
             if (has_next) make_plan(nxt, (k + 1) % 3, plan);
-            stage(q0, true, kc0, plan, false);
+            half2(acc, q0, true, kc0, plan, false);
         }
-        stage(q0 + nk - 1, false, kc1, plan, tail);
+        half1(acc, q0 + nk - 1, false, kc0, plan, tail);
+        half2(acc, q0 + nk - 1, false, kc1, plan, tail);
         if (!wm) ring_barrier();
-
-        // ---- epilogue: a lane of acc[a][b][i][j] holds D[weight row 4*kg + r of block j of weight half b][activation row
-        // row16 of block i of activation half a],
-        // i.e. 4 consecutive output columns of one row: one 8-byte store per (i, j) ----
-        const int m = cur.mt * kBM + wm * 64 + row16;
-        if (SPLIT && cur.part >= 0) {
-            // a piece of a split tile: the raw fp32 sums of its k-range, [activation row][weight row] of the tile
-            const int lane_e = lane_fresh(), row16 = lane_e & 15, kg = lane_e >> 4;
-            float* dst = p.partial + static_cast<size_t>(cur.part) * (kBM * kBN) + (wm * 64 + row16) * kBN + wn * 64 + kg * 4;
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    *reinterpret_cast<f32x4*>(dst + ((i >> 2) * 128 + (i & 3) * 16) * kBN + j * 16) = acc[i >> 2][j >> 1][i & 3][j & 1];
-        } else if (EPI == kSwiGLU) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int mi = m + (i >> 2) * 128 + (i & 3) * 16;
-                if (mi >= cur.ne) continue;
-                uint16_t* dst = p.out + static_cast<size_t>(cur.off + mi) * p.I;
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int col = cur.nt * 128 + wn * 32 + j * 16 + kg * 4;
-                    if (col >= p.I) continue;
-                    const f32x4 g = acc[i >> 2][0][i & 3][j], u = acc[i >> 2][1][i & 3][j];
-                    const uint32_t lo = f32_to_f16_bits(swiglu_fast(g[0], u[0])) |
-                                        (static_cast<uint32_t>(f32_to_f16_bits(swiglu_fast(g[1], u[1]))) << 16);
-                    const uint32_t hi = f32_to_f16_bits(swiglu_fast(g[2], u[2])) |
-                                        (static_cast<uint32_t>(f32_to_f16_bits(swiglu_fast(g[3], u[3]))) << 16);
-                    *reinterpret_cast<uint2*>(dst + col) = make_uint2(lo, hi);
-                }
-            }
-        } else {
-            // Whole-line stores: the wave's 128 x 64 sub-tile leaves as 16 instructions of 8 rows x 128 B. Row
-            // block i passes through the wave's own 2 KB of LDS (16 rows x 128 B; 16-byte granule g of row r at
-            // g ^ (r & 7)): lane (row16, kg) writes its four packed 4-column groups, then lane L reads granule
-            // L % 8 of row h * 8 + L / 8 (h = 0, 1). Stored straight from the MFMA layout (16 rows x 32 B per
-            // instruction) the epilogue cost ~100 us per DeepSeek-V2-Lite down launch (T = 16384, E = 64, K = 6).
-            uint8_t* stg = reinterpret_cast<uint8_t*>(lds) + tiled_epi_stage_offset(p.E) + wave * 2048;
-            const int lane_e = lane_fresh(), row16 = lane_e & 15, kg = lane_e >> 4;
-            const int rr = lane_e >> 3, gq = lane_e & 7;
-            const int col = cur.nt * kBN + wn * 64 + gq * 8;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const f32x4 v = acc[i >> 2][j >> 1][i & 3][j & 1];
-                    const uint32_t lo = f32_to_f16_bits(v[0]) | (static_cast<uint32_t>(f32_to_f16_bits(v[1])) << 16);
-                    const uint32_t hi = f32_to_f16_bits(v[2]) | (static_cast<uint32_t>(f32_to_f16_bits(v[3])) << 16);
-                    *reinterpret_cast<uint2*>(stg + row16 * 128 + (((2 * j + (kg >> 1)) ^ (row16 & 7)) << 4) + ((kg & 1) << 3)) =
-                        make_uint2(lo, hi);
-                }
-                // the reads take what other lanes of this wave just wrote (LDS operations of one wave run in order)
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                u32x4 v[2];
-#pragma unroll
-                for (int h = 0; h < 2; ++h) v[h] = *reinterpret_cast<const u32x4*>(stg + (h * 8 + rr) * 128 + ((gq ^ rr) << 4));
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // read before the next block's writes
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int r = (i >> 2) * 128 + wm * 64 + (i & 3) * 16 + h * 8 + rr;  // row of the tile
-                    if (cur.mt * kBM + r >= cur.ne || col >= p.H) continue;
-                    *reinterpret_cast<u32x4*>(p.out + static_cast<size_t>(rowtab[(k % 3) * kBM + r]) * p.H + col) = v[h];
-                }
-            }
-        }
+        epilogue(acc, cur, rowtab + (k % 3) * kBM);
+        // every lane of gate/up stores (past the buffer where there is no row), down skips blocks of rows or columns
+        // that are not there
+        stores = EPI == kSwiGLU ? 8 : (cur.ne - cur.mt * kBM >= kBM && (cur.nt + 1) * kBN <= p.H ? 16 : 0);
         if (!has_next) break;
         cur = nxt;
         q0 += nk;
