@@ -265,8 +265,13 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
             }
             t = xs.base + loc;
         }
-        int lo = T.e;  // the expert with tab[lo] <= t < tab[lo + 1], from the last tile's on
-        while (__builtin_amdgcn_readfirstlane(tab[lo + 1]) <= t) ++lo;
+        // the expert with tab[lo] <= t < tab[lo + 1], from the last tile's on: 64 experts a step (one LDS read, where a
+        // search one by one or by halves waits for up to E or log2(E) of them in turn)
+        int lo = T.e, past;
+        do {
+            past = __builtin_popcountll(__ballot(tab[min(lo + 1 + lane_fresh(), p.E)] <= t));
+            lo += past;
+        } while (past == kWave);
         T.e = lo;
         T.off = __builtin_amdgcn_readfirstlane(offs[lo]);
         T.ne = __builtin_amdgcn_readfirstlane(offs[lo + 1]) - T.off;
