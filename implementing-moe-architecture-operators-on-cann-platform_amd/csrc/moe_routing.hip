@@ -23,15 +23,8 @@
 // From 32768 tokens, for 32 < E <= 64 and H = 1024 or 2048, the resident kernel replaces the narrow one with the
 // same bits: one workgroup per CU holds the narrow kernel's w_gate fragments in registers and streams x through
 // an LDS ring, so w_gate is read once per CU instead of once per 32 tokens.
-// For E > 64 the rows kernel runs above 8192 tokens: a workgroup owns 64 tokens and each of its 4 waves 16 of them
-// over all of H, so the selection runs on the accumulators. w_gate stages (16 KB, row-major) are copied into LDS
-// with 16-byte direct-to-LDS loads and shared by the 4 waves; each wave's x rows stream through its own LDS ring
-// 16 k-steps ahead. Up to 8192 tokens the quarters kernel runs: a workgroup owns 16 tokens and each of its 4 waves
-// one quarter of H. Both add a token's H in the same four quarter sums, so the two give the same bits.
-// T = 16384, H = 2048: E = 256, K = 8 75.8 us; E = 128 39.0 us (the wide kernel below: 171.7 and 95.1 us). When w_gate cannot be copied 16 bytes at a time (E % 8 != 0, unaligned) the wide
-// kernel runs instead: its w_gate chunks are read with coalesced loads and written transposed, [expert][h], so a
-// lane's B fragment is one ds_read_b128; a stage of 2-4 chunks is loaded into registers while the previous one is
-// multiplied, two LDS buffers, one barrier per stage.
+// For E > 64 the direct kernel: a workgroup owns 16 to 64 tokens and each of its 4 waves one quarter of H; w_gate goes
+// from memory into registers and is transposed there, the quarters' sums meet in LDS.
 // HBM traffic per launch: T*H*2 (x) + H*E*2 (w_gate, L2-resident after the first workgroups) + T*K*6 bytes.
 
 #include <type_traits>
@@ -495,444 +488,200 @@ __global__ __launch_bounds__(waves_for(EB, TB) * kWave) void routing_topk_kernel
     }
 }
 
-constexpr int kWideTokens = 64;  // tokens per workgroup of the wide kernel
-constexpr int kWideWaves = 4;    // one 16-token MFMA row block each
+// The H reduction for E > 64: the k-steps of 32 fall into four quarters, each summed in k order from zero, and the
+// quarter sums are added as ((q0 + q1) + q2) + q3. A quarter is a whole number of stages of row_stage_ksteps(EB)
+// k-steps, quarter j = stages [j nst / 4, (j + 1) nst / 4), the last one with the k-step left over, if any. A token's
+// logits, ids and weights depend on nothing else, so they are the same in any batch and from any kernel.
+__host__ __device__ __forceinline__ int quarter_begin(int j, int nst) { return j * nst / 4; }
+constexpr int row_stage_ksteps(int eb) { return eb >= 16 ? 1 : 16 / eb; }
 
-// chunks of 32 h per stage (one memory round trip per stage), sized to ~64 registers of staged w_gate per lane
-constexpr int wide_chunks(int eb) { return eb == 8 ? 4 : 2; }
-constexpr int wide_pitch(int eb) { return wide_chunks(eb) * 32 + 8; }  // halfs per transposed row (16 B padding)
+// ---- direct kernel: E > 64 ----
+// One workgroup owns 16 TB tokens, wave j of its 4 sums quarter j of H for all experts. No LDS on the way of w_gate:
+// an MFMA wants 8 consecutive h of one expert from a lane, and a lane here loads 16 bytes (8 experts) of 8
+// consecutive rows h, so the 8 x 8 transposition stays within the lane (one v_perm_b32 per register). Lane
+// (n, kg) holds experts 128 s + 8 n + j, j < 8, of rows 8 kg .. 8 kg + 7: MFMA j of set s covers the experts
+// {128 s + 8 n + j} for n < 16, and each load instruction reads 4 rows x 256 bytes. The loads run in a register ring
+// of U units (a unit is one k-step of one set: 8 instructions, 8 KB a wave), U units ahead.
+// A row's last chunk is moved back to end with the row (start = E - 8), so E need not be a multiple of 8; experts it
+// shares with the chunk before are dropped. AL: 16-byte aligned rows (E % 8 == 0 and w_gate aligned); otherwise the
+// same 16-byte loads at 2-byte alignment.
+// What bounds it: a CU reads all of w_gate (3.7 MB at E = 256, H = 7168) at its 64 B/clk, about 27 us there whatever
+// T is (one workgroup alone takes 35 us), and from a few workgroups per XCD on they meet on the same L2 lines. The
+// kernels it replaces copied w_gate through LDS and read it back transposed, with one 16 KB stage in flight per wave
+// (up to 8192 tokens), shared a stage between 4 waves behind a barrier (above), or transposed it with LDS stores
+// (E % 8 != 0, or H / 32 odd at E <= 128). Measured, those -> this one (us):
+//   E = 256, H = 7168, K = 8: T = 1 45 -> 35, T = 64 46 -> 39, T = 4096 56 -> 48, T = 8192 110 -> 60, T = 16384 216 -> 112
+//   E = 256, H = 2048, K = 8: T = 64 27 -> 19, T = 4096 30 -> 20, T = 8192 57 -> 28, T = 16384 76 -> 52
+//   E = 128, H = 4096, K = 8: T = 64 21 -> 19, T = 4096 24 -> 20, T = 16384 67 -> 46
+//   E = 80, H = 4640, K = 2, T = 2814 164 -> 20; E = 250, H = 2048, K = 8, T = 16384 172 -> 59;
+//   E = 65, H = 1056, K = 2, T = 300 51 -> 15
+// A ring of 6 or 8 units: 0-5 % slower; x loaded non-temporally: 15-45 % slower (a load takes half lines of x, the
+// other halves are wanted a k-step later); 64 tokens and 256 experts in one pass: 233 us at T = 16384 (spills).
+// The sums of the 4 waves meet in LDS, 4 expert blocks at a time; each wave adds TB of them in quarter order and
+// writes the logits in expert order for the selection (16 lanes a token, 4 tokens a wave at a time).
+constexpr int kDirectWaves = 4;
+constexpr int kDirectUnits = 4;
+// 64 tokens and 256 experts: two passes, or the sums (256 registers) and the ring spill
+constexpr int direct_sets_per_pass(int eb, int tb) { return tb == 4 ? 1 : eb / 8; }
+constexpr int kDirectPhase = 4;  // expert blocks of 16 exchanged at a time
+constexpr int direct_pitch(int eb) { return eb * 16 + 4; }  // floats per row of logits
+constexpr size_t direct_part_bytes(int tb) { return static_cast<size_t>(kDirectWaves) * tb * kDirectPhase * 1024; }
+constexpr size_t direct_lds_needed(int eb, int tb) {
+    return direct_part_bytes(tb) + static_cast<size_t>(16) * tb * direct_pitch(eb) * 4;
+}
 
-// EB in {8, 16}: expert blocks of 16 (E <= 16 * EB)
-template <int EB>
-__global__ __launch_bounds__(kWideWaves * kWave) void routing_wide_kernel(const uint16_t* __restrict__ x,
-                                                                           const uint16_t* __restrict__ w_gate,
-                                                                           int32_t* __restrict__ expert_ids,
-                                                                           uint16_t* __restrict__ weights, int T,
-                                                                           int H, int E, int K,
-                                                                           int32_t* __restrict__ counts,
-                                                                           int32_t* __restrict__ rank) {
-    constexpr int Epad = EB * 16;
-    constexpr int CH = wide_chunks(EB);
-    constexpr int P = wide_pitch(EB);
-    constexpr int kThreads = kWideWaves * kWave;
-    constexpr int kPer = (CH * 32 * Epad + kThreads - 1) / kThreads;  // w_gate elements per thread per stage
-    extern __shared__ __align__(16) uint16_t wt[];                   // [2][Epad][P] halfs, then logits
-    float* logits = reinterpret_cast<float*>(wt + 2 * Epad * P);     // [64 tokens][Epad] fp32
-    const int tid = static_cast<int>(threadIdx.x);
+struct __attribute__((packed, aligned(2))) U32x4Unaligned {
+    u32x4 v;
+};
+
+template <int EB, int TB, bool AL>
+__global__ __launch_bounds__(kDirectWaves * kWave, 1) void routing_direct_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w_gate, int32_t* __restrict__ expert_ids,
+    uint16_t* __restrict__ weights, int T, int H, int E, int K, int32_t* __restrict__ counts,
+    int32_t* __restrict__ rank) {
+    constexpr int SETS = EB / 8;                     // of 128 experts
+    constexpr int SP = direct_sets_per_pass(EB, TB);  // sets summed together; x is read once per pass
+    constexpr int U = kDirectUnits;                  // units in the register ring
+    constexpr int G = U / SP;                        // k-steps in the ring
+    static_assert(U % SP == 0 && SETS % SP == 0, "whole k-steps in the ring, whole passes");
+    extern __shared__ __align__(16) uint8_t lds[];
     const int lane = lane_id();
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int row = lane & 15, kg = lane >> 4;
-    const int t0 = static_cast<int>(blockIdx.x) * kWideTokens;
-    const int tok = min(t0 + wave * 16 + row, T - 1);  // rows past T read a valid row; results are dropped
-    const uint16_t* xrow = x + static_cast<size_t>(tok) * H + kg * 8;
-    const int nchunks = H / 32;
-    const int nstages = (nchunks + CH - 1) / CH;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const int n16 = lane & 15, kg = lane >> 4;
+    const int t0 = static_cast<int>(blockIdx.x) * (16 * TB);
+    const int nks = H / 32, nst = nks / row_stage_ksteps(EB);
+    const int kb = row_stage_ksteps(EB) * quarter_begin(wave, nst);
+    const int n = (wave == 3 ? nks : row_stage_ksteps(EB) * quarter_begin(wave + 1, nst)) - kb;  // k-steps of the quarter
 
-    // stage s of w_gate: rows 32*CH*s .. +32*CH, element q -> (h = q / E, e = q % E), coalesced along e;
-    // rows past H read as zero
-    uint16_t wv[kPer];
-    f16x8 xa[CH];
-    auto load_stage = [&](int st) {
-        const int h0 = st * CH * 32;
-        const int n = min(CH * 32, H - h0) * E;
+    const int rows = min(16 * TB, T - t0);
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(x + static_cast<size_t>(t0) * H), 0, rows * H * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t wrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w_gate), 0, H * E * 2, 0x00020000);
+    int xo[TB];  // rows past the batch are past the buffer: zeros
 #pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-            const int q = tid + j * kThreads;
-            wv[j] = q < n ? w_gate[static_cast<size_t>(h0) * E + q] : uint16_t{0};
-        }
+    for (int tb = 0; tb < TB; ++tb) xo[tb] = ((tb * 16 + n16) * H + kg * 8) * 2;
+    f32x4* part = reinterpret_cast<f32x4*>(lds);  // [wave][tb][block of the phase][lane]
+    float* logits = reinterpret_cast<float*>(lds + direct_part_bytes(TB));
+    constexpr int P = direct_pitch(EB);
+    for (int set0 = 0; set0 < SETS; set0 += SP) {
+        int wo[SP];  // byte offset of the lane's chunk in its first row
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            if (st * CH + c < nchunks) {
-                xa[c] = load_f16x8(xrow + h0 + c * 32);
-            } else {  // a chunk past H contributes nothing, whatever x holds (0 * inf would be NaN)
+        for (int s = 0; s < SP; ++s) wo[s] = (kg * 8 * E + min(128 * (set0 + s) + 8 * n16, E - 8)) * 2;
+        u32x4 wr[U][8];
+        f16x8 xr[G][TB];
+        auto load_w = [&](u32x4 (&r)[8], int s, int k) __attribute__((always_inline)) {  // k-step k of the quarter
+            const int row0 = (kb + min(k, n - 1)) * 32;  // past the quarter: its last k-step again, never used
 #pragma unroll
-                for (int q = 0; q < 8; ++q) xa[c][q] = static_cast<f16>(0.0f);
+            for (int i = 0; i < 8; ++i) {
+                if constexpr (AL) {
+                    r[i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wo[s], (row0 + i) * E * 2, 0);
+                } else {
+                    const char* p = reinterpret_cast<const char*>(w_gate) + static_cast<size_t>(row0 + i) * E * 2;
+                    r[i] = reinterpret_cast<const U32x4Unaligned*>(p + wo[s])->v;
+                }
             }
-        }
-    };
-    auto store_stage = [&](int buf) {
-        uint16_t* dst = wt + buf * Epad * P;
+        };
+        auto load_x = [&](f16x8 (&r)[TB], int k) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < kPer; ++j) {
-            const int q = tid + j * kThreads;
-            if (q < CH * 32 * E) dst[(q % E) * P + q / E] = wv[j];
-        }
-    };
-    // experts E..Epad-1 of both buffers read as zero
-    for (int i = tid; i < 2 * (Epad - E) * P; i += kThreads) {
-        const int b = i / ((Epad - E) * P), r = i % ((Epad - E) * P);
-        wt[b * Epad * P + E * P + r] = 0;
-    }
-
-    f32x4 acc[EB];
+            for (int tb = 0; tb < TB; ++tb)
+                r[tb] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(xrs, xo[tb], (kb + min(k, n - 1)) * 64, 0));
+        };
+        f32x4 acc[TB][SP * 8];
 #pragma unroll
-    for (int b = 0; b < EB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    load_stage(0);
-    store_stage(0);
-    f16x8 a[CH];
+        for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
-    for (int c = 0; c < CH; ++c) a[c] = xa[c];
-    __syncthreads();
-    for (int st = 0; st < nstages; ++st) {
-        const int buf = st & 1;
-        if (st + 1 < nstages) load_stage(st + 1);
-        const uint16_t* src = wt + buf * Epad * P + row * P + kg * 8;
+            for (int b = 0; b < SP * 8; ++b) acc[tb][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        auto step = [&](int g) __attribute__((always_inline)) {  // the ring's k-step g
 #pragma unroll
-        for (int c = 0; c < CH; ++c)
+            for (int s = 0; s < SP; ++s) {
+                const u32x4(&r)[8] = wr[g * SP + s];
 #pragma unroll
-            for (int b = 0; b < EB; ++b) {
-                const f16x8 bv = *reinterpret_cast<const f16x8*>(src + b * 16 * P + c * 32);
-                acc[b] = mfma16x16x32(a[c], bv, acc[b]);
+                for (int j = 0; j < 8; ++j) {
+                    u32x4 f;  // expert 8 n + j of the set, rows 8 kg .. 8 kg + 7
+#pragma unroll
+                    for (int p = 0; p < 4; ++p)
+                        f[p] = __builtin_amdgcn_perm(r[2 * p + 1][j >> 1], r[2 * p][j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
+#pragma unroll
+                    for (int tb = 0; tb < TB; ++tb)
+                        acc[tb][s * 8 + j] = mfma16x16x32(xr[g][tb], __builtin_bit_cast(f16x8, f), acc[tb][s * 8 + j]);
+                    if (j % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // else the fragments of a whole k-step are built at once
+                }
             }
-        if (st + 1 < nstages) {
-            store_stage(buf ^ 1);  // that buffer was last read in stage st - 1
+        };
+        if (n > 0) {
 #pragma unroll
-            for (int c = 0; c < CH; ++c) a[c] = xa[c];
+            for (int g = 0; g < G; ++g) {
+                load_x(xr[g], g);
+#pragma unroll
+                for (int s = 0; s < SP; ++s) load_w(wr[g * SP + s], s, g);
+            }
+            int k = 0;
+            for (; k + G <= n; k += G) {
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    step(g);
+                    load_x(xr[g], k + g + G);
+#pragma unroll
+                    for (int s = 0; s < SP; ++s) load_w(wr[g * SP + s], s, k + g + G);
+                    __builtin_amdgcn_sched_barrier(0);  // the loads leave here, not where the next iteration wants them
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < G - 1; ++g)
+                if (k + g < n) step(g);
         }
-        __syncthreads();
-    }
-    // D[token 4*kg + r][expert b*16 + row] of this wave's 16 tokens
-#pragma unroll
-    for (int b = 0; b < EB; ++b)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) logits[(wave * 16 + kg * 4 + r) * Epad + b * 16 + row] = acc[b][r];
-    __syncthreads();
 
-    // ---- 16 lanes per token (EB experts a lane), 4 tokens per wave at a time ----
-    constexpr int TPW = kWave / kSelLanes;
-    for (int tb = wave * TPW; tb < kWideTokens; tb += kWideWaves * TPW) {
-        const int t = tb + lane / kSelLanes;
-        const bool active = t0 + t < T;
-        select_row<EB>(logits + t * Epad, E, K, active, expert_ids + static_cast<size_t>(active ? t0 + t : 0) * K,
-                       weights + static_cast<size_t>(active ? t0 + t : 0) * K);
+        // ---- the quarters' sums in quarter order, into logits[token][expert] ----
+#pragma unroll
+        for (int ph = 0; ph < SP * 8 / kDirectPhase; ++ph) {
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                for (int bb = 0; bb < kDirectPhase; ++bb)
+                    part[((wave * TB + tb) * kDirectPhase + bb) * kWave + lane] = acc[tb][ph * kDirectPhase + bb];
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < TB; ++i) {
+                const int at = wave * TB + i, tb = at / kDirectPhase, b = set0 * 8 + ph * kDirectPhase + at % kDirectPhase;
+                f32x4 v = part[at * kWave + lane];
+#pragma unroll
+                for (int q = 1; q < kDirectWaves; ++q) v = v + part[(q * TB * kDirectPhase + at) * kWave + lane];
+                const int first = 128 * (b / 8) + 8 * n16;  // the chunk's own first expert
+                const int e = min(first, E - 8) + b % 8;
+                if (e >= first) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) logits[(tb * 16 + 4 * kg + r) * P + e] = v[r];
+                }
+            }
+            __syncthreads();
+        }
+    }
+    // ---- selection: 16 lanes a token ----
+#pragma unroll
+    for (int i = 0; i < TB; ++i) {
+        const int tl = i * 16 + wave * 4 + kg, t = t0 + tl;
+        const bool active = t < T;
+        const int tr = active ? t : 0;
+        select_row<EB>(logits + tl * P, E, K, active, expert_ids + static_cast<size_t>(tr) * K,
+                       weights + static_cast<size_t>(tr) * K);
     }
     // ---- optional tail: the block's slots ranked by expert, for the permute's scatter ----
     if (counts != nullptr) {
         __syncthreads();  // the block's ids are written and the logits are no longer read
-        constexpr int MAXIT = (kWideTokens * kRankTopK + kWideWaves * kWave - 1) / (kWideWaves * kWave);
-        rank_slots<kWideWaves, MAXIT>(expert_ids, t0 * K, min(T, t0 + kWideTokens) * K, E, counts_stride(E),
-                                      reinterpret_cast<int*>(logits),
-                                      counts + static_cast<size_t>(blockIdx.x) * counts_stride(E), rank);
-    }
-}
-
-// ---- the rows kernel: each wave owns 16 tokens over all of H, w_gate stages shared by the workgroup ----
-// A workgroup of kRowWaves waves routes kRowTokens tokens. Per stage of SK 32-row k-steps (16 KB of w_gate):
-//   * the four waves copy the stage's w_gate rows, in their own row-major layout (16-byte chunks XOR-swizzled by
-//     row), into a ring of kRowWStages shared LDS stages with 16-byte direct-to-LDS loads, three stages ahead,
-//     one barrier per stage;
-//   * each wave copies its 16 token rows of x (64 B per row and k-step) into its own LDS ring, kRowXDepth k-steps
-//     ahead of their use, so each CU keeps ~64 KB of x in flight without spending registers on it;
-//   * A fragments are ds_read_b128 from the x ring, B fragments two ds_read_b64_tr_b16 from the w_gate stage.
-// The k-steps of each quarter of H add in order (quarter_begin below). The kernel runs for E > 64 whenever its
-// copies can (E % 8 == 0, a 16-byte aligned w_gate, SK dividing H / 32) and T > 8192; the quarters kernel gives
-// the same bits below that, so a token's bits do not depend on its batch.
-// At E <= 64 it was slower than the narrow kernel (T = 16384, E = 64: 27.8 µs alone and 34.2 µs in the layer,
-// against 21.8 and 30.2 µs): every wave reads all of w_gate from LDS, four times the narrow kernel's share.
-// At few tokens each 16-token block multiplies all of w_gate on one CU, and the compiler's wait for every copy in
-// flight before a transposing read (see the quarters kernel) leaves the ring no deeper than one stage, so the time
-// does not fall with T: H = 7168, E = 256 (3.7 MB of w_gate) 140 µs at T = 1, 185 µs at T = 128 to 2048, where
-// the quarters kernel takes 44-55 µs. Measured before it and not kept: workgroups of 1 or 2 waves (16 or 32
-// tokens, more CUs) 137 / 145 µs at T = 128 but 385 / 362 µs at T = 16384; a 7-stage w_gate ring 187 µs; the
-// rows kernel double-buffered with each stage read whole before the next one's copies, as the quarters kernel
-// does, 192 µs at T = 128 and 2x slower at E = 128.
-// The selection then runs on the accumulators: the MFMA leaves lane (row kg = lane / 16, column n) with token
-// 4 kg + r, expert 16 b + n in acc[b][r], i.e. each 16-lane DPP row holds one token's experts as select_vals
-// wants them.
-// The H reduction of the rows and quarters kernels: the stages fall into four quarters (quarter j = stages
-// [j nst / 4, (j + 1) nst / 4)), each summed in k order from zero, and the quarter sums are added as
-// ((q0 + q1) + q2) + q3. The rows kernel sums the quarters one after the other in each wave; the quarters kernel
-// gives each quarter to a wave of its own. Both make the same fp32 operations for a token, so its logits, ids and
-// weights do not depend on which of them ran.
-__host__ __device__ __forceinline__ int quarter_begin(int j, int nst) { return j * nst / 4; }
-
-constexpr int kRowWaves = 4;
-constexpr int kRowTokens = 16 * kRowWaves;
-constexpr int kRowXDepth = 16;                                               // x k-steps in flight per wave
-constexpr int kRowWStages = 4;                                               // w_gate ring: 3 stages ahead
-constexpr int row_stage_ksteps(int eb) { return eb >= 16 ? 1 : 16 / eb; }   // 16 KB of w_gate per stage
-constexpr size_t row_lds_bytes(int eb) {
-    return kRowWStages * 16384 + static_cast<size_t>(kRowWaves) * (kRowXDepth + row_stage_ksteps(eb)) * 1024;
-}
-
-template <int EB>
-__global__ __launch_bounds__(kRowWaves * kWave) void routing_rows_kernel(const uint16_t* __restrict__ x,
-                                                                          const uint16_t* __restrict__ w_gate,
-                                                                          int32_t* __restrict__ expert_ids,
-                                                                          uint16_t* __restrict__ weights, int T,
-                                                                          int H, int E, int K,
-                                                                          int32_t* __restrict__ counts,
-                                                                          int32_t* __restrict__ rank) {
-    constexpr int Epad = EB * 16;
-    constexpr int SK = row_stage_ksteps(EB);
-    constexpr int NW = kRowWStages;       // w_gate ring slots; stage i + NW - 1 is copied while i is used
-    constexpr int NXS = kRowXDepth / SK;  // x stages issued ahead of the one in use (>= NW, see the wait below)
-    constexpr int XR = NXS + 1;           // x ring slots (stages) per wave
-    constexpr int kStage = SK * 32 * Epad * 2;
-    static_assert(kStage == 16384 && NXS >= NW && NW >= 2, "stage geometry");
-    extern __shared__ __align__(16) uint8_t lds[];
-    const int lane = lane_id();
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
-    uint8_t* wbuf = lds;                                          // [NW][kStage]
-    uint8_t* xbuf = lds + NW * kStage + wave * XR * SK * 1024;    // this wave's ring: [XR][SK][16 rows][64 B]
-    const int t0 = static_cast<int>(blockIdx.x) * kRowTokens;
-    const int nst = H / 32 / SK;  // the host runs this kernel only when SK divides H / 32
-
-    const __amdgpu_buffer_rsrc_t wrs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w_gate), 0, H * E * 2, 0x00020000);
-    // x rows of this workgroup's tokens only (at most kRowTokens rows: 32-bit offsets for any T)
-    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(x + static_cast<size_t>(t0) * H), 0, min(kRowTokens, T - t0) * H * 2, 0x00020000);
-    // x copy: lane -> row lane / 4 (token t0 + 16 wave + row, clamped into the batch), 16-byte chunk lane % 4
-    const int xoff = (min(wave * 16 + lane / 4, T - 1 - t0) * H + (lane % 4) * 8) * 2;
-    // w_gate copy: wave w fills 1 KB slabs w, w + 4, w + 8, w + 12 of a stage; lane -> 16-byte slot of the slab
-    int woff[4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        const int off = (wave + 4 * m) * 1024 + lane * 16;
-        const int R = off / (32 * EB), pc = (off % (32 * EB)) / 16;  // stage row (SK k-steps of 32), slot
-        const int c = pc ^ ((R % 32) & (2 * EB - 1));                 // the logical chunk stored in slot pc
-        woff[m] = (R * E + (c * 8 < E ? c * 8 : 0)) * 2;              // padding chunks copy any valid chunk
-    }
-    // fragment reads: A at row * 64 + kg * 16 of a k-step's x block; B as in the narrow kernel's LDS path
-    const int arow = lane & 15, kg = lane >> 4;
-    int frag_off[2][EB];
-    {
-        const int sl = lane & 15;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int b = 0; b < EB; ++b) {
-                const int r = 8 * kg + 4 * h + sl / 4;
-                const int e = 16 * b + 4 * (sl % 4);
-                frag_off[h][b] = wstage_chunk<EB>(r, e / 8) + (e % 8) * 2;
-            }
-    }
-    auto issue_w = [&](int st) __attribute__((always_inline)) {
-        uint8_t* dst = wbuf + (st % NW) * kStage;
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (__attribute__((address_space(3))) void*)(dst + (wave + 4 * m) * 1024),
-                                                     16, static_cast<int>(woff[m]), st * SK * 32 * E * 2, 0, 0);
-    };
-    auto issue_x = [&](int st) __attribute__((always_inline)) {
-#pragma unroll
-        for (int ks = 0; ks < SK; ++ks)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (__attribute__((address_space(3))) void*)(xbuf + ((st % XR) * SK + ks) * 1024),
-                                                     16, xoff, (st * SK + ks) * 64, 0, 0);
-    };
-
-    f32x4 acc[EB];   // the current quarter's sum
-    f32x4 qsum[EB];  // the finished quarters' sum, ((q0 + q1) + q2)
-#pragma unroll
-    for (int b = 0; b < EB; ++b) acc[b] = qsum[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // Issue order: x(0 .. NXS-1), w(0 .. NW-2), then per iteration j: w(j + NW - 1), x(j + NXS).
-    for (int st = 0; st < min(NXS, nst); ++st) issue_x(st);
-    for (int st = 0; st < min(NW - 1, nst); ++st) issue_w(st);
-    // The quarters run one after the other (the copies run on across their boundaries); each starts from zero and
-    // joins the sum when it ends.
-    int i = 0;
-    for (int j = 0; j < 4; ++j) {
-        for (const int iend = quarter_begin(j + 1, nst); i < iend; ++i) {
-            // This wave's copies of w_gate stage i and of x stage i have landed. After w(i) (iteration i - NW + 1, or
-            // the prologue) came x(i - NW + 1 + NXS) and then NW - 2 iterations of w + x: SK + (NW - 2)(4 + SK) copies
-            // when every one of them went out, i.e. when iteration i - 1 still issued both; otherwise wait for all.
-            // x(i) went out no later than iteration i - NXS <= i - NW, before w(i).
-            if (i >= NW - 1 && i + NW - 2 < nst && i - 1 + NXS < nst) {
-                __builtin_amdgcn_s_waitcnt(vmcnt_imm(SK + (NW - 2) * (4 + SK)));
-            } else {
-                __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-            }
-            __syncthreads();  // every wave's w(i) is visible; every wave is done with w(i - 1) and its x(i - 1)
-            if (i + NW - 1 < nst) issue_w(i + NW - 1);
-            if (i + NXS < nst) issue_x(i + NXS);
-            const uint8_t* ws = wbuf + (i % NW) * kStage;
-            const uint8_t* xs = xbuf + (i % XR) * SK * 1024;
-#pragma unroll
-            for (int ks = 0; ks < SK; ++ks) {
-                const f16x8 a = *reinterpret_cast<const f16x8*>(xs + ks * 1024 + arow * 64 + kg * 16);
-                const uint8_t* wk = ws + ks * 32 * Epad * 2;
-#pragma unroll
-                for (int b = 0; b < EB; ++b) {
-                    const s16x4 lo = lds_read_tr16(wk + frag_off[0][b]);
-                    const s16x4 hi = lds_read_tr16(wk + frag_off[1][b]);
-                    const f16x8 bv = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-                    acc[b] = mfma16x16x32(a, bv, acc[b]);
-                }
-            }
-        }
-        if (j < 3) {
-#pragma unroll
-            for (int b = 0; b < EB; ++b) {
-                qsum[b] = j == 0 ? acc[b] : qsum[b] + acc[b];
-                acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-        }
-    }
-#pragma unroll
-    for (int b = 0; b < EB; ++b) acc[b] = qsum[b] + acc[b];  // + q3
-    // ---- selection from the accumulators: round r routes token 4 kg + r of each DPP row ----
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        float v[EB];
-#pragma unroll
-        for (int b = 0; b < EB; ++b) v[b] = acc[b][r];
-        const int t = t0 + wave * 16 + 4 * kg + r;
-        const bool active = t < T;
-        const int tr = active ? t : 0;
-        select_vals<EB>(v, E, K, active, expert_ids + static_cast<size_t>(tr) * K, weights + static_cast<size_t>(tr) * K);
-    }
-    // ---- optional tail: the block's slots ranked by expert, for the permute's scatter ----
-    if (counts != nullptr) {
-        __syncthreads();  // the block's ids are written and the stages are no longer read
-        constexpr int MAXIT = (kRowTokens * kRankTopK + kRowWaves * kWave - 1) / (kRowWaves * kWave);
-        rank_slots<kRowWaves, MAXIT>(expert_ids, t0 * K, min(T, t0 + kRowTokens) * K, E, counts_stride(E),
-                                     reinterpret_cast<int*>(lds),
-                                     counts + static_cast<size_t>(blockIdx.x) * counts_stride(E), rank);
-    }
-}
-
-// ---- the quarters kernel: one 16-token block per workgroup, wave j sums quarter j of the stages ----
-// With few tokens the rows kernel's 64-token workgroups leave most CUs idle and every wave multiplies all of
-// w_gate. Here a workgroup owns 16 tokens and each of its 4 waves streams one quarter of the stages through
-// double-buffered stages of its own (w_gate 16 KB, x SK KB), with no barrier in the loop: a wave reads only what
-// its own copies wrote. The compiler waits for every direct-to-LDS copy in flight (vmcnt(0)) before a
-// ds_read_b64_tr_b16 that follows it, since it cannot tell which LDS bytes a copy writes, so a stage is read
-// whole into registers before the next stage's copies go out; those then land while the stage's MFMAs run.
-// Wave 0 then adds the other waves' sums in quarter order, ((q0 + q1) + q2) + q3 as the rows kernel does, and
-// selects.
-constexpr size_t quarter_lds_bytes(int eb) { return 4 * (2 * size_t(16384) + 2 * size_t(row_stage_ksteps(eb)) * 1024); }
-
-template <int EB>
-__global__ __launch_bounds__(4 * kWave) void routing_quarters_kernel(const uint16_t* __restrict__ x,
-                                                                     const uint16_t* __restrict__ w_gate,
-                                                                     int32_t* __restrict__ expert_ids,
-                                                                     uint16_t* __restrict__ weights, int T, int H,
-                                                                     int E, int K, int32_t* __restrict__ counts,
-                                                                     int32_t* __restrict__ rank) {
-    constexpr int Epad = EB * 16;
-    constexpr int SK = row_stage_ksteps(EB);
-    constexpr int kStage = SK * 32 * Epad * 2;
-    constexpr int kWaveLds = 2 * kStage + 2 * SK * 1024;
-    static_assert(kStage == 16384, "stage geometry");
-    extern __shared__ __align__(16) uint8_t lds[];
-    const int lane = lane_id();
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
-    uint8_t* wbuf = lds + wave * kWaveLds;  // [2][kStage]
-    uint8_t* xbuf = wbuf + 2 * kStage;       // [2][SK][16 rows][64 B]
-    const int t0 = static_cast<int>(blockIdx.x) * 16;
-    const int nst = H / 32 / SK;  // the host runs this kernel only when SK divides H / 32
-    const int s0 = quarter_begin(wave, nst);
-    const int n = quarter_begin(wave + 1, nst) - s0;  // this wave's stages: s0 .. s0 + n - 1
-
-    const __amdgpu_buffer_rsrc_t wrs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w_gate), 0, H * E * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(x + static_cast<size_t>(t0) * H), 0, min(16, T - t0) * H * 2, 0x00020000);
-    // x copy: lane -> row lane / 4 (token t0 + row, clamped into the batch), 16-byte chunk lane % 4
-    const int xoff = (min(lane / 4, T - 1 - t0) * H + (lane % 4) * 8) * 2;
-    // w_gate copy: the wave fills all 16 slabs of 1 KB of its stage; lane -> 16-byte slot of the slab
-    int woff[16];
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-        const int off = m * 1024 + lane * 16;
-        const int R = off / (32 * EB), pc = (off % (32 * EB)) / 16;  // stage row (SK k-steps of 32), slot
-        const int c = pc ^ ((R % 32) & (2 * EB - 1));                 // the logical chunk stored in slot pc
-        woff[m] = (R * E + (c * 8 < E ? c * 8 : 0)) * 2;              // padding chunks copy any valid chunk
-    }
-    const int arow = lane & 15, kg = lane >> 4;
-    int frag_off[2][EB];
-    {
-        const int sl = lane & 15;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int b = 0; b < EB; ++b) {
-                const int r = 8 * kg + 4 * h + sl / 4;
-                const int e = 16 * b + 4 * (sl % 4);
-                frag_off[h][b] = wstage_chunk<EB>(r, e / 8) + (e % 8) * 2;
-            }
-    }
-    auto issue = [&](int l) __attribute__((always_inline)) {  // this wave's stage s0 + l
-        uint8_t* dst = wbuf + (l & 1) * kStage;
-#pragma unroll
-        for (int m = 0; m < 16; ++m)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (__attribute__((address_space(3))) void*)(dst + m * 1024), 16,
-                                                     static_cast<int>(woff[m]), (s0 + l) * SK * 32 * E * 2, 0, 0);
-#pragma unroll
-        for (int ks = 0; ks < SK; ++ks)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (__attribute__((address_space(3))) void*)(xbuf + ((l & 1) * SK + ks) * 1024),
-                                                     16, xoff, ((s0 + l) * SK + ks) * 64, 0, 0);
-    };
-
-    f32x4 acc[EB];
-#pragma unroll
-    for (int b = 0; b < EB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (n > 0) issue(0);
-    for (int l = 0; l < n; ++l) {
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // this wave's copies of stage l (the only ones in flight)
-        const uint8_t* ws = wbuf + (l & 1) * kStage;
-        const uint8_t* xs = xbuf + (l & 1) * SK * 1024;
-        f16x8 a[SK], bv[SK][EB];
-#pragma unroll
-        for (int ks = 0; ks < SK; ++ks) {
-            a[ks] = *reinterpret_cast<const f16x8*>(xs + ks * 1024 + arow * 64 + kg * 16);
-            const uint8_t* wk = ws + ks * 32 * Epad * 2;
-#pragma unroll
-            for (int b = 0; b < EB; ++b) {
-                const s16x4 lo = lds_read_tr16(wk + frag_off[0][b]);
-                const s16x4 hi = lds_read_tr16(wk + frag_off[1][b]);
-                bv[ks][b] = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            }
-        }
-        // stage l + 1 refills the buffers of stage l - 1, whose reads fed MFMAs in the previous iteration
-        if (l + 1 < n) issue(l + 1);
-#pragma unroll
-        for (int ks = 0; ks < SK; ++ks)
-#pragma unroll
-            for (int b = 0; b < EB; ++b) acc[b] = mfma16x16x32(a[ks], bv[ks][b], acc[b]);
-    }
-    // waves 1-3 park their quarter sums in their own (idle) w_gate buffers: lane-major f32x4 per expert block
-    if (wave > 0) {
-#pragma unroll
-        for (int b = 0; b < EB; ++b) *reinterpret_cast<f32x4*>(wbuf + (b * kWave + lane) * 16) = acc[b];
-    }
-    __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-        for (int j = 1; j < 4; ++j)
-#pragma unroll
-            for (int b = 0; b < EB; ++b)
-                acc[b] = acc[b] + *reinterpret_cast<const f32x4*>(lds + j * kWaveLds + (b * kWave + lane) * 16);
-        // ---- selection from the sums: round r routes token 4 kg + r of each DPP row ----
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            float v[EB];
-#pragma unroll
-            for (int b = 0; b < EB; ++b) v[b] = acc[b][r];
-            const int t = t0 + 4 * kg + r;
-            const bool active = t < T;
-            const int tr = active ? t : 0;
-            select_vals<EB>(v, E, K, active, expert_ids + static_cast<size_t>(tr) * K,
-                            weights + static_cast<size_t>(tr) * K);
-        }
-    }
-    // ---- optional tail: the block's slots ranked by expert, for the permute's scatter ----
-    if (counts != nullptr) {
-        __syncthreads();  // the block's ids are written and the sums are no longer read
-        constexpr int MAXIT = (16 * kRankTopK + 4 * kWave - 1) / (4 * kWave);
-        rank_slots<4, MAXIT>(expert_ids, t0 * K, min(T, t0 + 16) * K, E, counts_stride(E), reinterpret_cast<int*>(lds),
-                             counts + static_cast<size_t>(blockIdx.x) * counts_stride(E), rank);
+        constexpr int MAXIT = (16 * TB * kRankTopK + kDirectWaves * kWave - 1) / (kDirectWaves * kWave);
+        rank_slots<kDirectWaves, MAXIT>(expert_ids, t0 * K, min(T, t0 + 16 * TB) * K, E, counts_stride(E),
+                                        reinterpret_cast<int*>(lds),
+                                        counts + static_cast<size_t>(blockIdx.x) * counts_stride(E), rank);
     }
 }
 
 // ---- split routing of one 16-token block (moe_layer, E > 64, T <= 16) ----
-// At T <= 16 the quarters kernel's one workgroup reads all of w_gate on one CU (3.7 MB at E = 256, H = 7168:
-// ~50 us). Here workgroup (j, g) runs quarter j of the quarters kernel's k-steps for the kSplitGB expert blocks
+// At T <= 16 the direct kernel's one workgroup reads all of w_gate on one CU (3.7 MB at E = 256, H = 7168:
+// 35 us). Here workgroup (j, g) runs quarter j of the direct kernel's k-steps for the kSplitGB expert blocks
 // of group g only (one wave), and writes its fp32 sums to the layer's workspace; a second launch adds the
-// quarters as the quarters kernel does, ((q0 + q1) + q2) + q3, and selects. Every expert's sum runs the same
-// MFMAs on the same fragments in the same k order, so ids and weights are the quarters kernel's bit for bit; only
+// quarters as the direct kernel does, ((q0 + q1) + q2) + q3, and selects. Every expert's sum runs the same
+// MFMAs on the same fragments in the same k order, so ids and weights are the direct kernel's bit for bit; only
 // the staging differs (a window of 16 kSplitGB experts, stages of kSplitSK k-steps).
 constexpr int kSplitGB = 2;
 constexpr int kSplitSK = row_stage_ksteps(kSplitGB);  // 8 k-steps of 32 rows x 32 experts: 16 KB per stage
@@ -952,7 +701,7 @@ __global__ __launch_bounds__(kWave) void routing_split_partial_kernel(const uint
     const int lane = lane_id();
     const int j = static_cast<int>(blockIdx.x) % 4, grp = static_cast<int>(blockIdx.x) / 4;
     const int e0 = grp * Gpad;  // first expert of the window
-    // quarter j of the quarters kernel's k-steps (its stages hold row_stage_ksteps(EB) k-steps each); the host
+    // quarter j of the direct kernel's k-steps (its stages hold row_stage_ksteps(EB) k-steps each); the host
     // runs this kernel only where SK divides every quarter
     constexpr int SKq = row_stage_ksteps(EB);
     const int nstq = H / 32 / SKq;
@@ -962,7 +711,7 @@ __global__ __launch_bounds__(kWave) void routing_split_partial_kernel(const uint
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w_gate), 0, H * E * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, T * H * 2, 0x00020000);
     const int xoff = (min(lane / 4, T - 1) * H + (lane % 4) * 8) * 2;
-    // w_gate copy: the quarters kernel's stage layout for GB blocks, columns e0 .. e0 + Gpad - 1 of each row
+    // w_gate copy: the narrow kernel's stage layout (wstage_chunk) for GB blocks, columns e0 .. e0 + Gpad - 1 of each row
     int woff[16];
 #pragma unroll
     for (int m = 0; m < 16; ++m) {
@@ -1027,7 +776,7 @@ __global__ __launch_bounds__(kWave) void routing_split_partial_kernel(const uint
         *reinterpret_cast<f32x4*>(part + ((static_cast<size_t>(j) * EB + grp * GB + b) * kWave + lane) * 4) = acc[b];
 }
 
-// the quarters' sums in the quarters kernel's order, then its selection
+// the quarters' sums in the direct kernel's order, then its selection
 template <int EB>
 __global__ __launch_bounds__(kWave) void routing_split_select_kernel(const float* __restrict__ part,
                                                                      int32_t* __restrict__ expert_ids,
@@ -1296,25 +1045,6 @@ __global__ __launch_bounds__(kResWaves * kWave) void routing_resident_kernel(con
     }
 }
 
-size_t wide_lds_bytes(int eb) {
-    const int pitch = eb == 8 ? wide_pitch(8) : wide_pitch(16);
-    return static_cast<size_t>(2) * eb * 16 * pitch * sizeof(uint16_t) +
-           static_cast<size_t>(kWideTokens) * eb * 16 * sizeof(float);
-}
-
-template <int EB>
-hipError_t launch_wide(const uint16_t* x, const uint16_t* w_gate, int32_t* ids, uint16_t* w, int T, int H, int E,
-                       int K, int32_t* counts, int32_t* rank, hipStream_t stream) {
-    const int grid = (T + kWideTokens - 1) / kWideTokens;
-    const size_t lds = wide_lds_bytes(EB);
-    const hipError_t attr = ensure_lds_limit(reinterpret_cast<const void*>(&routing_wide_kernel<EB>),
-                                             static_cast<int>(lds));
-    if (attr != hipSuccess) return attr;
-    TraceScope trace("moe_routing_topk", stream);
-    routing_wide_kernel<EB><<<grid, kWideWaves * kWave, lds, stream>>>(x, w_gate, ids, w, T, H, E, K, counts, rank);
-    return hipGetLastError();
-}
-
 template <int EB, int TB, bool LW, bool NTX>
 hipError_t launch_narrow_nt(const uint16_t* x, const uint16_t* w_gate, int32_t* ids, uint16_t* w, int T, int H, int E,
                             int K, int32_t* counts, int32_t* rank, hipStream_t stream) {
@@ -1381,44 +1111,41 @@ hipError_t launch_resident(const uint16_t* x, const uint16_t* w_gate, int32_t* i
 // virtual wave; whole 1024-column ring slots, the fragments within 128 VGPRs).
 bool resident_shape(int H, int eb) { return eb == kResEB && (H == 1024 || H == 2048); }
 
-template <int EB>
-hipError_t launch_quarters(const uint16_t* x, const uint16_t* w_gate, int32_t* ids, uint16_t* w, int T, int H, int E,
-                           int K, int32_t* counts, int32_t* rank, hipStream_t stream) {
-    const int grid = (T + 15) / 16;
-    const size_t lds = quarter_lds_bytes(EB);
-    const hipError_t attr = ensure_lds_limit(reinterpret_cast<const void*>(&routing_quarters_kernel<EB>),
-                                             static_cast<int>(lds));
+template <int EB, int TB, bool AL>
+hipError_t launch_direct(const uint16_t* x, const uint16_t* w_gate, int32_t* ids, uint16_t* w, int T, int H, int E,
+                         int K, int32_t* counts, int32_t* rank, size_t lds, hipStream_t stream) {
+    const void* fn = reinterpret_cast<const void*>(&routing_direct_kernel<EB, TB, AL>);
+    const hipError_t attr = ensure_lds_limit(fn, 160 * 1024);
     if (attr != hipSuccess) return attr;
     TraceScope trace("moe_routing_topk", stream);
-    routing_quarters_kernel<EB><<<grid, 4 * kWave, lds, stream>>>(x, w_gate, ids, w, T, H, E, K, counts, rank);
+    routing_direct_kernel<EB, TB, AL><<<(T + 16 * TB - 1) / (16 * TB), kDirectWaves * kWave, lds, stream>>>(
+        x, w_gate, ids, w, T, H, E, K, counts, rank);
     return hipGetLastError();
 }
 
-template <int EB>
-hipError_t launch_rows(const uint16_t* x, const uint16_t* w_gate, int32_t* ids, uint16_t* w, int T, int H, int E,
-                       int K, int32_t* counts, int32_t* rank, hipStream_t stream) {
-    const int grid = (T + kRowTokens - 1) / kRowTokens;
-    const size_t lds = row_lds_bytes(EB);
-    const hipError_t attr = ensure_lds_limit(reinterpret_cast<const void*>(&routing_rows_kernel<EB>),
-                                             static_cast<int>(lds));
-    if (attr != hipSuccess) return attr;
-    TraceScope trace("moe_routing_topk", stream);
-    routing_rows_kernel<EB><<<grid, kRowWaves * kWave, lds, stream>>>(x, w_gate, ids, w, T, H, E, K, counts, rank);
-    return hipGetLastError();
+template <int EB, int TB>
+hipError_t launch_direct(const uint16_t* x, const uint16_t* w_gate, int32_t* ids, uint16_t* w, int T, int H, int E,
+                         int K, int32_t* counts, int32_t* rank, size_t lds, hipStream_t stream) {
+    return narrow_lds_weights(w_gate, H, E)
+               ? launch_direct<EB, TB, true>(x, w_gate, ids, w, T, H, E, K, counts, rank, lds, stream)
+               : launch_direct<EB, TB, false>(x, w_gate, ids, w, T, H, E, K, counts, rank, lds, stream);
 }
 
-// Which kernel routes: the narrow kernel for E <= 64; for E > 64 the rows kernel when its copies can run (lw:
-// w_gate rows can be copied 16 bytes at a time, and whole stages of k-steps), else the wide kernel. The choice
-// does not depend on T, so a token's ids and weights do not depend on the batch it is routed in.
-enum RoutingKernel { kNarrowKernel, kWideKernel, kRowsKernel, kQuartersKernel, kResidentKernel };
-// Tokens up to which the quarters kernel runs instead of the rows kernel (same bits). The rows kernel takes about
-// the same time from T = 128 to 16384 (one workgroup per CU at most, each streaming all of w_gate): 215.6, 75.8,
-// 66.5 and 39.0 us at T = 16384 for the four shapes below. The quarters kernel (us):
-//   E = 256, H = 7168, K = 8: T = 128 46.9, 8192 113.8, 12288 167.0, 16384 220.6
-//   E = 256, H = 2048, K = 8: T = 4096 30.7, 8192 58.9, 12288 86.0, 16384 113.0
-//   E = 128, H = 4096, K = 8: T = 8192 47.0, 12288 69.3, 16384 91.0
-//   E = 128, H = 2048, K = 6: T = 8192 32.0, 12288 46.6, 16384 61.7
-constexpr int64_t kQuartersMaxTokens = 8192;
+// Which kernel routes: the narrow kernel for E <= 64 (or the resident kernel, same bits), the direct kernel above.
+enum RoutingKernel { kNarrowKernel, kResidentKernel, kDirectKernel };
+// Token blocks of 16 per workgroup of the direct kernel, see there: 1 while that makes one round of the CUs (256), then
+// as many as keep w_gate's reads per CU down.
+int direct_token_blocks(int T, int eb) { return T > 8192 ? 4 : (T > 4096 && eb == 16 ? 2 : 1); }
+// The LDS a launch reserves: the exchange of the sums and the logits fit in it; a CU holds one workgroup (its waves
+// use most of the register file) whatever it is.
+size_t direct_lds_bytes(int eb, int tb, bool lw) {
+    if (tb < 4) return 4 * (2 * size_t(16384) + 2 * size_t(row_stage_ksteps(eb)) * 1024);
+    if (lw) return 4 * size_t(16384) + 4 * (16 + size_t(row_stage_ksteps(eb))) * 1024;
+    return eb == 8 ? 100 * 1024 : 136 * 1024;
+}
+static_assert(direct_lds_needed(8, 4) <= 100 * 1024 && direct_lds_needed(16, 4) <= 4 * 16384 + 4 * 17 * 1024 &&
+                  direct_lds_needed(16, 2) <= 4 * (2 * 16384 + 2 * 1024),
+              "the direct kernel's LDS");
 // Tokens from which 32 < E <= 64 routes through the resident kernel (same bits as the narrow kernel). Isolated
 // launches at H = 2048, E = 64, K = 6, x streamed from HBM (non-temporal) / evicted first, us:
 //   T =  4096: narrow 12.2 / 14.9,  resident 13.6 / 17.8
@@ -1432,10 +1159,8 @@ constexpr int64_t kResidentMinTokens = 32768;
 static_assert(kResidentMinTokens * 1024 * 2 >= kNtXBytes, "the resident kernel always loads x non-temporally");
 RoutingKernel routing_kernel(int T, int H, int E, bool lw) {
     const int eb = routing_expert_blocks(E);
-    if (eb <= 4) return lw && T >= kResidentMinTokens && resident_shape(H, eb) ? kResidentKernel : kNarrowKernel;
-    const bool rows_ok = lw && (H / 32) % row_stage_ksteps(eb) == 0;
-    if (!rows_ok) return kWideKernel;
-    return T <= kQuartersMaxTokens ? kQuartersKernel : kRowsKernel;
+    if (eb > 4) return kDirectKernel;
+    return lw && T >= kResidentMinTokens && resident_shape(H, eb) ? kResidentKernel : kNarrowKernel;
 }
 
 template <int EB>
@@ -1453,8 +1178,8 @@ hipError_t launch_split(const uint16_t* x, const uint16_t* w_gate, int32_t* ids,
 }  // namespace
 
 bool routing_split_applies(int T, int H, int E, bool lw) {
-    if (T < 1 || T > 16 || routing_kernel(T, H, E, lw) != kQuartersKernel) return false;
     const int skq = row_stage_ksteps(routing_expert_blocks(E)), nst = H / 32 / skq;
+    if (T < 1 || T > 16 || E <= 64 || !lw || H / 32 % skq != 0) return false;
     for (int j = 0; j < 4; ++j)
         if (skq * (quarter_begin(j + 1, nst) - quarter_begin(j, nst)) % kSplitSK != 0) return false;
     return true;
@@ -1484,30 +1209,24 @@ bool routing_lds_weights(const void* w_gate, int H, int E) { return narrow_lds_w
 int routing_tokens_per_block(int T, int H, int E, bool lw) {
     const int eb = routing_expert_blocks(E);
     switch (routing_kernel(T, H, E, lw)) {
-        case kRowsKernel: return kRowTokens;
-        case kQuartersKernel: return 16;
         case kResidentKernel: return 16 * res_blocks_per_wg(T);
-        case kWideKernel: return kWideTokens;
+        case kDirectKernel: return 16 * direct_token_blocks(T, eb);
         default: return kTokensPerBlock * narrow_token_blocks(T, eb);
     }
 }
 int routing_block_threads(int T, int H, int E, bool lw) {
     const int eb = routing_expert_blocks(E);
     switch (routing_kernel(T, H, E, lw)) {
-        case kRowsKernel: return kRowWaves * kWave;
-        case kQuartersKernel: return 4 * kWave;
         case kResidentKernel: return kResWaves * kWave;
-        case kWideKernel: return kWideWaves * kWave;
+        case kDirectKernel: return kDirectWaves * kWave;
         default: return waves_for(eb, narrow_token_blocks(T, eb)) * kWave;
     }
 }
 int routing_lds_bytes(int T, int H, int E, bool lw) {
     const int eb = routing_expert_blocks(E);
     switch (routing_kernel(T, H, E, lw)) {
-        case kRowsKernel: return static_cast<int>(row_lds_bytes(eb));
-        case kQuartersKernel: return static_cast<int>(quarter_lds_bytes(eb));
         case kResidentKernel: return static_cast<int>(kResLdsBytes);
-        case kWideKernel: return static_cast<int>(wide_lds_bytes(eb));
+        case kDirectKernel: return static_cast<int>(direct_lds_bytes(eb, direct_token_blocks(T, eb), lw));
         default: return static_cast<int>(narrow_lds_bytes(eb, narrow_token_blocks(T, eb), lw));
     }
 }
@@ -1519,13 +1238,18 @@ int routing_blocks(int T, int H, int E, bool lw) {
 hipError_t launch_routing_topk(const uint16_t* x, const uint16_t* w_gate, int32_t* ids, uint16_t* w, int T, int H,
                                int E, int K, hipStream_t stream, int32_t* counts, int32_t* rank) {
     const int eb = routing_expert_blocks(E);
-    switch (routing_kernel(T, H, E, narrow_lds_weights(w_gate, H, E))) {
-        case kRowsKernel:
-            return eb == 8 ? launch_rows<8>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream)
-                           : launch_rows<16>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream);
-        case kQuartersKernel:
-            return eb == 8 ? launch_quarters<8>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream)
-                           : launch_quarters<16>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream);
+    const bool lw = narrow_lds_weights(w_gate, H, E);
+    switch (routing_kernel(T, H, E, lw)) {
+        case kDirectKernel: {
+            const int tb = direct_token_blocks(T, eb);
+            const size_t lds = direct_lds_bytes(eb, tb, lw);
+            if (eb == 8)
+                return tb == 1 ? launch_direct<8, 1>(x, w_gate, ids, w, T, H, E, K, counts, rank, lds, stream)
+                               : launch_direct<8, 4>(x, w_gate, ids, w, T, H, E, K, counts, rank, lds, stream);
+            return tb == 1   ? launch_direct<16, 1>(x, w_gate, ids, w, T, H, E, K, counts, rank, lds, stream)
+                   : tb == 2 ? launch_direct<16, 2>(x, w_gate, ids, w, T, H, E, K, counts, rank, lds, stream)
+                             : launch_direct<16, 4>(x, w_gate, ids, w, T, H, E, K, counts, rank, lds, stream);
+        }
         case kResidentKernel:
             return H == 1024 ? launch_resident<4>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream)
                              : launch_resident<8>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream);
@@ -1534,9 +1258,7 @@ hipError_t launch_routing_topk(const uint16_t* x, const uint16_t* w_gate, int32_
     switch (eb) {
         case 1: return launch_eb<1>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream);
         case 2: return launch_eb<2>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream);
-        case 4: return launch_eb<4>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream);
-        case 8: return launch_wide<8>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream);
-        default: return launch_wide<16>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream);
+        default: return launch_eb<4>(x, w_gate, ids, w, T, H, E, K, counts, rank, stream);
     }
 }
 

@@ -1429,3 +1429,30 @@ def test_tiled_tile_and_stage_edges(ops, H, I):
                          rng.standard_normal((E, I, H), dtype=np.float32) / math.sqrt(I)], axis=1).astype(np.float16)
     eo = f32(host(ops.MoeExpertFFN(dev(x), dev(ids), dev(w), dev(ew))))
     within(oracle.compare(eo, oracle_ffn_threads(f32(x), ids, f32(ew), I)), max_abs=2**-6, mean_abs=2**-10, cos=0.9999)
+
+
+@pytest.mark.parametrize("H,E,K", [
+    (32, 72, 3),     # one k-step: three of the four quarters of H are empty
+    (96, 250, 8),    # E % 8 != 0: the row's last 8 experts overlap the chunk before; 3 k-steps
+    (1056, 80, 2),   # 33 k-steps of 32 at two a stage: one left over for the last quarter
+    (2080, 129, 5),  # one expert past 128
+    (544, 256, 200),  # K above the 16 lanes of a token
+])
+def test_routing_direct_kernel(ops, H, E, K):
+    """E > 64: a token's ids and weights are the same bits with 16, 32 (E > 128) or 64 tokens per workgroup (T up to
+    4096, up to 8192 and above), and with w_gate rows that are not 16-byte aligned; the small batch also against the
+    oracle's routing."""
+    T = 8195
+    rng = np.random.default_rng(H + E)
+    x = rng.standard_normal((T, H)).astype(np.float16)
+    wg = (rng.standard_normal((H, E)) / math.sqrt(H)).astype(np.float16)
+    x_d, wg_d = dev(x), dev(wg)
+    ids_all, w_all = (host(v) for v in ops.MoeRoutingTopK(x_d, wg_d, K))
+    ids, w = (host(v) for v in ops.MoeRoutingTopK(x_d[:301].contiguous(), wg_d, K))
+    check_routing(ids, w, x[:301], wg, K, f"direct H{H} E{E} K{K}")
+    buf = torch.empty(H * E + 1, dtype=torch.float16, device="cuda")
+    odd = buf[1:].view(H, E)  # 2-byte aligned only
+    odd.copy_(wg_d)
+    others = [ops.MoeRoutingTopK(x_d[:4700].contiguous(), wg_d, K), ops.MoeRoutingTopK(x_d[:301].contiguous(), odd, K)]
+    for i, v in [(ids_all, w_all)] + [tuple(host(o) for o in p) for p in others]:
+        assert np.array_equal(i[:301], ids) and np.array_equal(v[:301].view(np.uint16), w.view(np.uint16))
