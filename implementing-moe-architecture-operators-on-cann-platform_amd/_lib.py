@@ -91,6 +91,8 @@ _lib: C.CDLL | None = None
 def load() -> C.CDLL:
     """Load the library once; raises RuntimeError if it was not built."""
     global _lib
+    if _lib is not None:  # set once, after every signature is
+        return _lib
     with _lock:
         if _lib is None:
             if not LIB_PATH.exists():

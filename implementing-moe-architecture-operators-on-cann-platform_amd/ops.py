@@ -7,6 +7,11 @@ queued on `stream` (torch's current stream when None). Outputs and any workspace
 allocated while that stream is current, so torch's caching allocator ties them to the stream the kernels run
 on: a workspace freed on return cannot be handed to other work before those kernels have finished with it.
 Errors raise MoeError with the library's message, before anything is launched.
+
+A call's own host work is kept to a few microseconds: at decode sizes the kernels of an operator take 5-10 us, and
+asking the library for every shape and entering a stream context took longer than that (T = 8, H = 64, E = 4,
+I = 256, the three operators: 60 us of host time, now 25, of which the four launches take ~13). Shapes that fit are worked out here, any other goes to the library's infer
+function, which words the error; the stream context is entered only for a stream that the caller names.
 """
 from __future__ import annotations
 
@@ -21,23 +26,31 @@ from ._lib import MoeError, check, dims
 _TORCH_DT = {_lib.DT_FLOAT16: torch.float16, _lib.DT_INT32: torch.int32}
 
 
-def _stream(stream) -> "torch.cuda.Stream":
-    return stream if stream is not None else torch.cuda.current_stream()
-
-
 def _stream_ptr(stream) -> int:
-    return int(_stream(stream).cuda_stream)
+    """The raw stream a call runs on: `stream`, or the current stream of the current device."""
+    if stream is not None:
+        return int(stream.cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+_CURRENT = contextlib.nullcontext()
+
+
+def _on(stream):
+    """Allocations made within belong to the stream the kernels run on."""
+    return _CURRENT if stream is None else torch.cuda.stream(stream)
 
 
 def _need(t: torch.Tensor, name: str, dtype: torch.dtype) -> None:
+    if isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == dtype and t.is_contiguous():
+        return
     if not isinstance(t, torch.Tensor):
         raise MoeError(1, f"{name} must be a tensor")
     if t.device.type != "cuda":
         raise MoeError(4, f"{name} must be a device tensor (got {t.device})")
     if t.dtype != dtype:
         raise MoeError(4, f"{name} must be {dtype} (got {t.dtype})")
-    if not t.is_contiguous():
-        raise MoeError(4, f"{name} must be contiguous (ND format)")
+    raise MoeError(4, f"{name} must be contiguous (ND format)")
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -83,18 +96,42 @@ def layer_workspace_bytes(T: int, H: int, E: int, K: int, I: int) -> int:
     return int(_lib.load().moe_layer_workspace_bytes(T, H, E, K, I))
 
 
+def _routing_shape(x, w_gate, topK):
+    """[T, K] of the routing outputs (the rules of moe_routing_topk_infer_shape)."""
+    xs, gs = x.shape, w_gate.shape
+    if len(xs) == 2 and len(gs) == 2 and xs[1] == gs[0] and type(topK) is int:
+        k = topK if topK > 0 else 2
+        if k <= gs[1]:
+            return xs[0], k
+    return infer_routing(tuple(xs), tuple(gs), topK)[0][0]
+
+
+def _ffn_inter(x, ids_shape, expert_weights, intermediateSize) -> int:
+    """The intermediate size of the expert FFN (the rules of moe_expert_ffn_infer_shape)."""
+    xs, es = x.shape, expert_weights.shape
+    if (len(xs) == 2 and len(ids_shape) == 2 and len(es) == 3 and ids_shape[0] == xs[0] and es[2] == xs[1]
+            and es[1] % 3 == 0 and type(intermediateSize) is int):
+        inter = es[1] // 3
+        if intermediateSize <= 0 or intermediateSize == inter:
+            return inter
+    return infer_expert_ffn(tuple(xs), tuple(ids_shape), tuple(es), intermediateSize)[2]
+
+
+def _bytes(workspace: torch.Tensor) -> int:
+    return workspace.numel() * workspace.element_size()
+
+
 def MoeRoutingTopK(x: torch.Tensor, w_gate: torch.Tensor, topK: int = 2, stream=None):
     """x[T,H] fp16, w_gate[H,E] fp16 -> (expert_ids[T,K] int32, weights[T,K] fp16)."""
     _need(x, "x", torch.float16)
     _need(w_gate, "w_gate", torch.float16)
-    (ids_shape, ids_dt), (w_shape, w_dt) = infer_routing(tuple(x.shape), tuple(w_gate.shape), topK)
-    s = _stream(stream)
-    with torch.cuda.stream(s):
-        ids = torch.empty(ids_shape, dtype=ids_dt, device=x.device)
-        w = torch.empty(w_shape, dtype=w_dt, device=x.device)
-    T, H = x.shape
-    check(_lib.load().moe_routing_topk(x.data_ptr(), w_gate.data_ptr(), ids.data_ptr(), w.data_ptr(), T, H,
-                                       w_gate.shape[1], ids_shape[1], int(s.cuda_stream)))
+    T, K = shape = _routing_shape(x, w_gate, topK)
+    H, E = w_gate.shape
+    with _on(stream):
+        ids = x.new_empty(shape, dtype=torch.int32)
+        w = x.new_empty(shape)
+    check(_lib.load().moe_routing_topk(x.data_ptr(), w_gate.data_ptr(), ids.data_ptr(), w.data_ptr(), T, H, E, K,
+                                       _stream_ptr(stream)))
     return ids, w
 
 
@@ -105,20 +142,18 @@ def MoeExpertFFN(x: torch.Tensor, expert_ids: torch.Tensor, weights: torch.Tenso
     _need(expert_ids, "expert_ids", torch.int32)
     _need(weights, "weights", torch.float16)
     _need(expert_weights, "expert_weights", torch.float16)
-    out_shape, out_dt, inter = infer_expert_ffn(tuple(x.shape), tuple(expert_ids.shape),
-                                                tuple(expert_weights.shape), intermediateSize)
+    inter = _ffn_inter(x, expert_ids.shape, expert_weights, intermediateSize)
     T, H = x.shape
     E, K = expert_weights.shape[0], expert_ids.shape[1]
-    need = workspace_bytes(T, H, E, K, inter)
-    s = _stream(stream)
-    with torch.cuda.stream(s):
+    lib = _lib.load()
+    with _on(stream):
         if workspace is None:
-            workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
-        expert_out = torch.empty(out_shape, dtype=out_dt, device=x.device)
-    check(_lib.load().moe_expert_ffn(x.data_ptr(), expert_ids.data_ptr(), weights.data_ptr(),
-                                     expert_weights.data_ptr(), expert_out.data_ptr(), workspace.data_ptr(),
-                                     workspace.numel() * workspace.element_size(), T, H, E, K, inter,
-                                     int(s.cuda_stream)))
+            need = int(lib.moe_expert_ffn_workspace_bytes(T, H, E, K, inter))
+            workspace = x.new_empty(max(need, 1), dtype=torch.uint8)
+        expert_out = x.new_empty((T, K, H))
+    check(lib.moe_expert_ffn(x.data_ptr(), expert_ids.data_ptr(), weights.data_ptr(), expert_weights.data_ptr(),
+                             expert_out.data_ptr(), workspace.data_ptr(), _bytes(workspace), T, H, E, K, inter,
+                             _stream_ptr(stream)))
     return expert_out
 
 
@@ -131,15 +166,16 @@ def MoeCombine(expert_out: torch.Tensor, expert_ids: torch.Tensor | None, weight
     _need(weights, "weights", torch.float16)
     if expert_ids is not None:
         _need(expert_ids, "expert_ids", torch.int32)
-    y_shape, y_dt = infer_combine(tuple(expert_out.shape), tuple(expert_ids.shape) if expert_ids is not None else None)
-    T, K, H = expert_out.shape
-    if tuple(weights.shape) != (T, K):
+    es = expert_out.shape
+    if len(es) != 3 or (expert_ids is not None and expert_ids.shape != es[:2]):
+        infer_combine(tuple(es), tuple(expert_ids.shape) if expert_ids is not None else None)  # raises
+    T, K, H = es
+    if weights.shape != es[:2]:
         raise MoeError(3, f"weights shape {tuple(weights.shape)} != {(T, K)}")
-    s = _stream(stream)
-    with torch.cuda.stream(s):
-        y = torch.empty(y_shape, dtype=y_dt, device=expert_out.device)
+    with _on(stream):
+        y = expert_out.new_empty((T, H))
     check(_lib.load().moe_combine(expert_out.data_ptr(), _ptr(expert_ids), weights.data_ptr(), y.data_ptr(), T, H, K,
-                                  int(s.cuda_stream)))
+                                  _stream_ptr(stream)))
     return y
 
 
@@ -152,23 +188,22 @@ def MoeExpertFFNCombine(x: torch.Tensor, expert_ids: torch.Tensor, weights: torc
     _need(expert_ids, "expert_ids", torch.int32)
     _need(weights, "weights", torch.float16)
     _need(expert_weights, "expert_weights", torch.float16)
-    out_shape, out_dt, inter = infer_expert_ffn(tuple(x.shape), tuple(expert_ids.shape),
-                                                tuple(expert_weights.shape), intermediateSize)
+    inter = _ffn_inter(x, expert_ids.shape, expert_weights, intermediateSize)
     T, H = x.shape
     E, K = expert_weights.shape[0], expert_ids.shape[1]
-    if tuple(weights.shape) != (T, K):
+    if weights.shape != expert_ids.shape:
         raise MoeError(3, f"weights shape {tuple(weights.shape)} != {(T, K)}")
-    need = workspace_bytes(T, H, E, K, inter)
-    s = _stream(stream)
-    with torch.cuda.stream(s):
+    lib = _lib.load()
+    with _on(stream):
         if workspace is None:
-            workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
-        expert_out = torch.empty(out_shape, dtype=out_dt, device=x.device)
-        y = torch.empty((T, H), dtype=torch.float16, device=x.device)
-    check(_lib.load().moe_expert_ffn_combine(x.data_ptr(), expert_ids.data_ptr(), weights.data_ptr(),
-                                             expert_weights.data_ptr(), expert_out.data_ptr(), y.data_ptr(),
-                                             workspace.data_ptr(), workspace.numel() * workspace.element_size(), T,
-                                             H, E, K, inter, int(s.cuda_stream)))
+            need = int(lib.moe_expert_ffn_workspace_bytes(T, H, E, K, inter))
+            workspace = x.new_empty(max(need, 1), dtype=torch.uint8)
+        expert_out = x.new_empty((T, K, H))
+        y = x.new_empty((T, H))
+    check(lib.moe_expert_ffn_combine(x.data_ptr(), expert_ids.data_ptr(), weights.data_ptr(),
+                                     expert_weights.data_ptr(), expert_out.data_ptr(), y.data_ptr(),
+                                     workspace.data_ptr(), _bytes(workspace), T, H, E, K, inter,
+                                     _stream_ptr(stream)))
     return expert_out, y
 
 
@@ -189,24 +224,21 @@ def moe_layer_fused(x: torch.Tensor, w_gate: torch.Tensor, expert_weights: torch
     _need(x, "x", torch.float16)
     _need(w_gate, "w_gate", torch.float16)
     _need(expert_weights, "expert_weights", torch.float16)
-    (ids_shape, ids_dt), (w_shape, w_dt) = infer_routing(tuple(x.shape), tuple(w_gate.shape), topK)
-    out_shape, out_dt, inter = infer_expert_ffn(tuple(x.shape), ids_shape, tuple(expert_weights.shape),
-                                                intermediateSize)
-    T, H = x.shape
-    E, K = expert_weights.shape[0], ids_shape[1]
-    need = layer_workspace_bytes(T, H, E, K, inter)
-    s = _stream(stream)
-    with torch.cuda.stream(s):
+    T, K = shape = _routing_shape(x, w_gate, topK)
+    inter = _ffn_inter(x, shape, expert_weights, intermediateSize)
+    H, E = x.shape[1], expert_weights.shape[0]
+    lib = _lib.load()
+    with _on(stream):
         if workspace is None:
-            workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
-        ids = torch.empty(ids_shape, dtype=ids_dt, device=x.device)
-        w = torch.empty(w_shape, dtype=w_dt, device=x.device)
-        expert_out = torch.empty(out_shape, dtype=out_dt, device=x.device)
-        y = torch.empty((T, H), dtype=torch.float16, device=x.device)
-    check(_lib.load().moe_layer(x.data_ptr(), w_gate.data_ptr(), expert_weights.data_ptr(), ids.data_ptr(),
-                                w.data_ptr(), expert_out.data_ptr(), y.data_ptr(), workspace.data_ptr(),
-                                workspace.numel() * workspace.element_size(), T, H, E, K, inter,
-                                int(s.cuda_stream)))
+            need = int(lib.moe_layer_workspace_bytes(T, H, E, K, inter))
+            workspace = x.new_empty(max(need, 1), dtype=torch.uint8)
+        ids = x.new_empty(shape, dtype=torch.int32)
+        w = x.new_empty(shape)
+        expert_out = x.new_empty((T, K, H))
+        y = x.new_empty((T, H))
+    check(lib.moe_layer(x.data_ptr(), w_gate.data_ptr(), expert_weights.data_ptr(), ids.data_ptr(), w.data_ptr(),
+                        expert_out.data_ptr(), y.data_ptr(), workspace.data_ptr(), _bytes(workspace), T, H, E, K,
+                        inter, _stream_ptr(stream)))
     return y, ids, w, expert_out
 
 

@@ -298,3 +298,32 @@ def test_package_fails_loudly_without_library(tmp_path, monkeypatch):
     monkeypatch.setattr(lib_mod, "_lib", None)
     with pytest.raises(RuntimeError, match="no\\s+CPU fallback"):
         lib_mod.load()
+
+
+def test_shape_rules_match_infer_functions(lib):
+    """ops works out the shapes of a fitting call itself: over fitting and unfitting ranks, sizes and attributes the
+    result, or the error, is the library's infer function's."""
+    import itertools
+
+    import torch
+
+    ops = package().ops
+
+    def outcome(fn):
+        try:
+            return fn()
+        except (lib_mod.MoeError, C.ArgumentError) as err:
+            return type(err), str(err)
+
+    def empty(shape):
+        return torch.empty(shape, device="meta")
+
+    xs = [(9, 64), (0, 64), (9, 32), (9, 64, 1), (64,)]
+    for x, g, k in itertools.product(xs, [(64, 8), (32, 8), (64,), (64, 1)], [2, 3, 8, 9, 1, 0, -4, True, 1.5]):
+        got = outcome(lambda: tuple(ops._routing_shape(empty(x), empty(g), k)))
+        assert got == outcome(lambda: ops.infer_routing(x, g, k)[0][0]), (x, g, k)
+    for x, ids, ew, inter in itertools.product(xs, [(9, 3), (0, 3), (9,), (9, 3, 1)],
+                                               [(8, 96, 64), (8, 97, 64), (8, 96, 32), (96, 64)],
+                                               [0, 32, 64, -1, True, 0.5]):
+        got = outcome(lambda: ops._ffn_inter(empty(x), ids, empty(ew), inter))
+        assert got == outcome(lambda: ops.infer_expert_ffn(x, ids, ew, inter)[2]), (x, ids, ew, inter)
