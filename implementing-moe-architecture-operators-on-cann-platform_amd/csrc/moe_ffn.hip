@@ -45,10 +45,30 @@ size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 //                                         112 rows 612.5 / 468.1 (experts above 128 rows take a second pass)
 //   H = 4096, E = 8,  K = 2, I = 14336    80 rows 726.7 / 784.0, 96 rows 779.1 / 804.8, 112 rows 1143.3 / 822.5
 // Shapes the wide kernels cannot run switch to the tiled schedule at 32 rows.
+// Expert weights of at least 1 GB (streamed from HBM whichever schedule runs, for long enough that the tiled one's
+// permute and fix-up launches do not show) switch earlier: the tiled kernels then cost the same from ~32 to ~100 rows
+// per expert, and with many or unevenly loaded experts the wide kernels' time is that of the fullest ones. The FFN
+// (wide / tiled, us, one box; Zipf = Zipf-skewed routing):
+//   H = 2048, E = 16, K = 2, I = 8192     56 rows 357.1 / 363.8, 64 rows 358.9 / 362.3, 72 rows 383.7 / 373.1,
+//                                         96 rows 427.6 / 373.1
+//   H = 4096, E = 8,  K = 2, I = 14336    40 rows 561.2 / 601.3, 56 rows 637.2 / 618.3, 72 rows 684.1 / 620.1
+//   H = 2048, E = 64, K = 6, I = 1408     32 rows 236.8 / 236.4, 40 rows 243.8 / 234.3, 56 rows 266.5 / 239.1
+//   H = 4096, E = 128, K = 8, I = 1536    40 rows 905.5 / 889.5, 56 rows 1043.4 / 923.9, 70 rows 1143.0 / 947.2
+//   H = 7168, E = 256, K = 8, I = 2048    37 rows 4156.6 / 4165.7, 60 rows 5365.6 / 4348.2
+//   H = 1024, E = 64, K = 4, I = 3072     37 rows 254.5 / 258.5, 50 rows 284.5 / 263.7
+//   Zipf: H = 2048, E = 16, I = 8192 72 rows 758.6 / 431.0; H = 2048, E = 64, I = 1408 37 rows 482.4 / 237.6
+// Below 1 GB the lines above hold (H = 1024, E = 96, K = 4, I = 1024: 40 rows 146.8 / 181.3; H = 1536, E = 12, K = 2,
+// I = 6144: 66 rows 203.1 / 231.6; H = 1024, E = 32, K = 4, I = 4096: 65 rows 197.7 / 205.1). Calls
+// without the split leftover round's workspace (splits.tiled off) and sizes past the tiled kernels' offsets keep them
+// too.
 constexpr int64_t kTiledMinRowsPerExpert = 32;
 constexpr int64_t kWideMaxRowsPerExpert = 97;
 constexpr int64_t kWideMaxRowsSmallI = 72;
 constexpr int64_t kWideLargeI = 4096;
+constexpr int64_t kLargeWeightBytes = int64_t{1} << 30;
+constexpr int64_t kManyExperts = 64;
+constexpr int64_t kLargeTiledMinRowsMany = 40;  // from kManyExperts experts
+constexpr int64_t kLargeTiledMinRows = 66;
 
 }  // namespace
 
@@ -57,6 +77,9 @@ int ffn_schedule(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, FfnSplit
     const int64_t wide_limit = I >= kWideLargeI ? kWideMaxRowsPerExpert : kWideMaxRowsSmallI;
     const int64_t limit = stream_wide_supported(static_cast<int>(H), static_cast<int>(I)) ? wide_limit
                                                                                           : kTiledMinRowsPerExpert;
+    if (splits.tiled && 6 * E * I * H >= kLargeWeightBytes &&
+        T * K >= (E >= kManyExperts ? kLargeTiledMinRowsMany : kLargeTiledMinRows) * E && tiled_supported(T, H, E, K, I))
+        return 1;
     const bool many_rows = T * K >= limit * E;
     if (tiled_shape_supported(H, E, I) && (many_rows || !stream_ok))
         return tiled_size_supported(T, H, K, I) ? 1 : -1;

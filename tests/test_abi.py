@@ -327,3 +327,17 @@ def test_shape_rules_match_infer_functions(lib):
                                                [0, 32, 64, -1, True, 0.5]):
         got = outcome(lambda: ops._ffn_inter(empty(x), ids, empty(ew), inter))
         assert got == outcome(lambda: ops.infer_expert_ffn(x, ids, ew, inter)[2]), (x, ids, ew, inter)
+
+
+@pytest.mark.parametrize("T,H,E,K,I,schedule", [
+    (1055, 2048, 16, 1, 8192, 0),  # 1.6 GB of expert weights, E < 64: tiled from 66 rows per expert
+    (1056, 2048, 16, 1, 8192, 1),
+    (426, 2048, 64, 6, 1408, 0),   # 1.1 GB, E >= 64: tiled from 40 rows
+    (427, 2048, 64, 6, 1408, 1),
+    (560, 1024, 16, 2, 512, 0),    # 50 MB, 70 rows: wide to 72 rows
+    (16384, 65536, 256, 1, 128, 0),  # 64 rows, but x reaches 2 GiB: still streamed, as below 72 rows before
+])
+def test_large_weights_switch_to_tiled_earlier(lib, T, H, E, K, I, schedule):
+    fp = lib_mod.FfnPlan()
+    assert lib.moe_expert_ffn_plan(T, H, E, K, I, C.byref(fp)) == MOE_OK
+    assert fp.schedule == schedule
