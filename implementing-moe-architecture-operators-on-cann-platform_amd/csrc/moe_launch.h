@@ -75,6 +75,7 @@ FfnWorkspace ffn_workspace_carve(void* base, int64_t T, int64_t H, int64_t E, in
 
 int permute_block_threads();
 int permute_chunks(int S);
+int permute_grid(int S, int E);  // workgroups of launch_permute's first launch
 size_t permute_scratch_bytes(int S, int E);
 hipError_t prepare_permute(int S, int E);  // kernel attributes, before the first launch of a call
 // the scatter alone, over chunk counts and ranks some other kernel wrote (counts rows of counts_stride(E) ints,

@@ -15,6 +15,8 @@
 //            a scan over the experts gives offsets[e], a scan over its own chunks each chunk's base, and slot s
 //            of expert e in chunk c goes to sorted_slot[offsets[e] + (e's slots in chunks before c) + rank[s]].
 //            Workgroup 0 writes offsets.
+// Few slots (permute_single) whose ids come from the caller (no routing tail) are sorted by one workgroup in one launch,
+// with counts and ranks in LDS and registers (permute_single_kernel).
 // No atomics and no cleared memory, so the result is deterministic and needs no memset before the call.
 // Slots whose id is outside [0, E) belong to no expert; the scatter workgroups write zeros into their expert_out
 // rows, each over its own chunks.
@@ -165,10 +167,121 @@ __global__ __launch_bounds__(kScatterThreads) void permute_scatter_kernel(
     }
 }
 
+// The whole sort of S <= kSingleSlots slots in workgroup 0: wave w takes the R consecutive slots from w R, 64 at a
+// time; lanes with the same id find each other with ballots over the id's bits, so a slot's place among the wave's
+// earlier slots of its expert is a popcount, and a running count per (wave, expert) in LDS carries it on. Exclusive
+// sums over the waves and over the experts then give every slot its row. The other workgroups write zeros into the
+// expert_out rows of ids outside [0, E). Latency bound: one round trip for the ids, ~25 instructions per 64 slots,
+// three barriers. Two launches -> this (us):
+//   S = 800, E = 8 12.3 -> 5.1; S = 2000, E = 16 12.2 -> 4.9; S = 4096, E = 16 12.0 -> 5.5; S = 4097, E = 40 11.4 -> 6.8
+//   S = 9003, E = 24 11.7 -> 9.5; S = 9186, E = 64 11.4 -> 10.4; S = 12288, E = 16 12.1 -> 10.9, E = 128 11.2 -> 14.5
+// The time grows with the slots times the id bits, so the line lies at 64 K of those (permute_single).
+constexpr int kSingleThreads = 1024;
+constexpr int kSingleWaves = kSingleThreads / kWave;
+constexpr int kSingleIters = 12;
+constexpr int kSingleSlots = kSingleThreads * kSingleIters;
+template <int MAXIT>
+__global__ __launch_bounds__(kSingleThreads) void permute_single_kernel(const int32_t* __restrict__ ids, int S, int E,
+                                                                        int H, int32_t* __restrict__ offsets,
+                                                                        int32_t* __restrict__ sorted_slot,
+                                                                        uint16_t* __restrict__ expert_out) {
+    __shared__ int wcnt[kSingleWaves * kMaxE];  // [wave][expert]: slots, then those of the waves before
+    __shared__ int offs[kMaxE];
+    const int tid = static_cast<int>(threadIdx.x);
+    if (blockIdx.x > 0) {
+        const int s = (static_cast<int>(blockIdx.x) - 1) * kSingleThreads + tid;
+        const int e = s < S ? ids[s] : 0;
+        if (e < 0 || e >= E) {
+            u32x4* row = reinterpret_cast<u32x4*>(expert_out + static_cast<size_t>(s) * H);
+            for (int j = 0; j < H / 8; ++j) row[j] = u32x4{0u, 0u, 0u, 0u};
+        }
+        return;
+    }
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = lane_id();
+    const int R = (S + kSingleThreads - 1) / kSingleThreads * kWave;  // at most 64 MAXIT
+    const int b0 = wave * R, b1 = min(S, b0 + R);
+    int e[MAXIT], r[MAXIT];
+#pragma unroll
+    for (int it = 0; it < MAXIT; ++it) {
+        const int s = b0 + it * kWave + lane;
+        e[it] = s < b1 ? ids[s] : -1;
+    }
+    for (int i = tid; i < kSingleWaves * E; i += kSingleThreads) wcnt[i] = 0;
+    __syncthreads();
+    const int nbits = 32 - __builtin_clz(max(1, E - 1));
+    const uint64_t below = (uint64_t{1} << lane) - 1;
+#pragma unroll
+    for (int it = 0; it < MAXIT; ++it) {
+        r[it] = 0;
+        if (b0 + it * kWave >= b1) continue;  // uniform: the wave's slots have ended
+        const bool valid = e[it] >= 0 && e[it] < E;
+        uint64_t same = __ballot(valid);
+        for (int b = 0; b < nbits; ++b) {
+            const bool bit = (e[it] >> b) & 1;
+            const uint64_t m = __ballot(bit);
+            same &= bit ? m : ~m;
+        }
+        const int before = __popcll(same & below);
+        if (valid) {
+            r[it] = wcnt[wave * E + e[it]] + before;
+            // the lane of each expert's first slot advances the count; every lane's read above is issued first
+            if (before == 0) wcnt[wave * E + e[it]] += __popcll(same);
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {  // totals and their exclusive sums, 64 experts at a time
+        int carry = 0;
+        for (int x0 = 0; x0 < E; x0 += kWave) {
+            const int x = x0 + lane;
+            int tot = 0;
+            if (x < E) {
+                int c[kSingleWaves];
+#pragma unroll
+                for (int w = 0; w < kSingleWaves; ++w) c[w] = wcnt[w * E + x];
+#pragma unroll
+                for (int w = 0; w < kSingleWaves; ++w) {
+                    wcnt[w * E + x] = tot;
+                    tot += c[w];
+                }
+            }
+            int incl = tot;
+#pragma unroll
+            for (int d = 1; d < kWave; d <<= 1) {
+                const int v = __shfl_up(incl, d, kWave);
+                if (lane >= d) incl += v;
+            }
+            if (x < E) {
+                offs[x] = carry + incl - tot;
+                offsets[x] = carry + incl - tot;
+            }
+            carry += __shfl(incl, kWave - 1, kWave);
+        }
+        if (lane == 0) offsets[E] = carry;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < MAXIT; ++it) {
+        const int s = b0 + it * kWave + lane;
+        if (s < b1 && e[it] >= 0 && e[it] < E) sorted_slot[offs[e[it]] + wcnt[wave * E + e[it]] + r[it]] = s;
+    }
+}
+
+}  // namespace
+
+namespace {
+int id_bits(int E) {
+    int bits = 1;
+    while ((1 << bits) < E) ++bits;
+    return bits;
+}
+bool permute_single(int S, int E) { return S <= kSingleSlots && S * id_bits(E) <= 65536; }
 }  // namespace
 
 int permute_block_threads() { return kThreads; }
 int permute_chunks(int S) { return (S + kChunk - 1) / kChunk; }
+int permute_grid(int S, int E) {
+    return permute_single(S, E) ? 1 + (S + kSingleThreads - 1) / kSingleThreads : permute_chunks(S);
+}
 
 // rank [S] i32, then (16-byte aligned) counts [chunks][counts_stride(E)] i32
 size_t permute_scratch_bytes(int S, int E) {
@@ -200,6 +313,15 @@ hipError_t launch_permute_scatter(const int32_t* ids, int S, int E, int H, const
 
 hipError_t launch_permute(const int32_t* ids, int S, int E, int H, FfnWorkspace ws, uint16_t* expert_out,
                           hipStream_t stream) {
+    if (permute_single(S, E)) {
+        TraceScope trace("moe_permute", stream);
+        const int grid = permute_grid(S, E);
+        if (S <= kSingleThreads * 4)
+            permute_single_kernel<4><<<grid, kSingleThreads, 0, stream>>>(ids, S, E, H, ws.offsets, ws.sorted_slot, expert_out);
+        else
+            permute_single_kernel<kSingleIters><<<grid, kSingleThreads, 0, stream>>>(ids, S, E, H, ws.offsets, ws.sorted_slot, expert_out);
+        return hipGetLastError();
+    }
     const int nchunks = permute_chunks(S);
     int32_t* rank = ws.pscratch;
     int32_t* counts = ws.pscratch + counts_stride(S);  // 16-byte aligned rows

@@ -1456,3 +1456,21 @@ def test_routing_direct_kernel(ops, H, E, K):
     others = [ops.MoeRoutingTopK(x_d[:4700].contiguous(), wg_d, K), ops.MoeRoutingTopK(x_d[:301].contiguous(), odd, K)]
     for i, v in [(ids_all, w_all)] + [tuple(host(o) for o in p) for p in others]:
         assert np.array_equal(i[:301], ids) and np.array_equal(v[:301].view(np.uint16), w.view(np.uint16))
+
+
+@pytest.mark.parametrize("S,E", [(80, 1), (1023, 8), (1025, 3), (4096, 13), (4097, 40), (8192, 100), (8193, 110),
+                                 (12288, 16), (12289, 16)])
+def test_permute_slot_counts(ops, S, E):
+    """The permute of a caller's ids, at the edges of its one-launch form (up to 64 K slots x id bits, 12288 slots; 4
+    or 12 rounds of 1024 slots): offsets and sorted_slot equal a stable sort, rows of ids outside [0, E) are zero."""
+    H, I = 96, 96
+    assert ffn_schedule(S, H, E, 1, I) == 1
+    rng = np.random.default_rng(S + E)
+    ids = rng.integers(0, E, (S, 1)).astype(np.int32)
+    bad = rng.choice(S, 5, replace=False)
+    ids[bad, 0] = [-1, E, E + 7, -2**31, 2**31 - 1]
+    x, w = rng.standard_normal((S, H)).astype(np.float16), np.ones((S, 1), np.float16)
+    ew = (rng.standard_normal((E, 3 * I, H)) / math.sqrt(H)).astype(np.float16)
+    eo_d, ws = run_ffn(ops, dev(x), dev(ids), dev(w), dev(ew), I)
+    check_permute(host(ws), ids, E)
+    assert not host(eo_d)[bad].any()
