@@ -38,8 +38,8 @@
 //   persistent   one workgroup per CU walks its tiles back to back and the ring runs on across them: the
 //                copies of a tile's first two stages go out during the previous tile's last two. The tile table
 //                (per-expert tile prefix and row offsets) is built once per workgroup in LDS, so finding a tile
-//                is a short search from the last tile's expert on; the next tile's 256 sorted-slot entries are copied into LDS a tile
-//                ahead.
+//                is a short search from the last tile's expert on; the next tile's 256 sorted-slot
+//                entries are copied into LDS a tile ahead.
 //   split        (down) the down projection has only ~2 tiles per CU at prefill, so a count-based schedule
 //                leaves the last round mostly idle: the tiles left over after the full rounds are split over k
 //                into pieces, one per workgroup, that write fp32 partial tiles; ffn_tiled_fixup_kernel adds them
@@ -90,8 +90,8 @@ constexpr int kMaxParts = 256;
 constexpr int kFixThreads = 256;
 constexpr int kFixRows = 16;  // tile rows per fix-up workgroup
 // The split pays off only while the leftover round is a large share of the down projection: at DeepSeek-V2-Lite
-// prefill (T = 16384, E = 64, K = 6, 13-14 rounds of 22-stage tiles) the unsplit kernel takes 575 us against
-// 589 us + a 15 us fix-up split; at 2-2.5 rounds (T = 8192, E = 16; Mixtral T = 4096) the split saves 100-215 us.
+// prefill (T = 16384, E = 64, K = 6, 13-14 rounds of 22-stage tiles) the kernel before the ticks took 575 us unsplit
+// against 589 us + a 15 us fix-up split (not timed again since); at 2-2.5 rounds (T = 8192, E = 16; Mixtral T = 4096) the split saves 100-215 us.
 constexpr int kSplitMaxRounds = 4;
 
 struct TiledArgs {
