@@ -226,7 +226,9 @@ def moe_layer_fused(x: torch.Tensor, w_gate: torch.Tensor, expert_weights: torch
     _need(expert_weights, "expert_weights", torch.float16)
     T, K = shape = _routing_shape(x, w_gate, topK)
     inter = _ffn_inter(x, shape, expert_weights, intermediateSize)
-    H, E = x.shape[1], expert_weights.shape[0]
+    H, E = w_gate.shape
+    if expert_weights.shape[0] != E:  # the library takes one E: it would read w_gate past its end or at another stride
+        raise MoeError(3, f"w_gate routes to {E} experts, expert_weights holds {expert_weights.shape[0]}")
     lib = _lib.load()
     with _on(stream):
         if workspace is None:

@@ -341,3 +341,28 @@ def test_large_weights_switch_to_tiled_earlier(lib, T, H, E, K, I, schedule):
     fp = lib_mod.FfnPlan()
     assert lib.moe_expert_ffn_plan(T, H, E, K, I, C.byref(fp)) == MOE_OK
     assert fp.schedule == schedule
+
+
+def test_fused_layer_takes_as_many_experts_as_it_routes_to(monkeypatch):
+    """moe_layer reads H * E of w_gate with the E of expert_weights: ops.moe_layer_fused refuses a w_gate of fewer
+    columns (its end would be read past) or of more (the rows would be read at the wrong stride) before it calls the
+    library. The library is replaced here, so nothing is launched."""
+    import types
+
+    import torch
+
+    ops = package().ops
+    calls = []
+    stub = types.SimpleNamespace(moe_layer_workspace_bytes=lambda *a: 64,
+                                 moe_layer=lambda *a: calls.append(a) or MOE_OK)
+    monkeypatch.setattr(ops, "_need", lambda *a: None)
+    monkeypatch.setattr(ops, "_stream_ptr", lambda stream: 0)
+    monkeypatch.setattr(ops._lib, "load", lambda: stub)
+    x, ew = torch.zeros((3, 64), dtype=torch.float16), torch.zeros((8, 96, 64), dtype=torch.float16)
+    for E in (7, 9, 16, 2):
+        with pytest.raises(lib_mod.MoeError) as err:
+            ops.moe_layer_fused(x, torch.zeros((64, E), dtype=torch.float16), ew, 2)
+        assert err.value.status == ERR_SHAPE
+        assert not calls
+    ops.moe_layer_fused(x, torch.zeros((64, 8), dtype=torch.float16), ew, 2)
+    assert len(calls) == 1
