@@ -144,6 +144,42 @@ FfnWorkspace ffn_workspace_carve(void* base, int64_t T, int64_t H, int64_t E, in
     return ws;
 }
 
+namespace {
+
+// Without the partial tiles of the split leftover round: the schedule lines below 1 GB of expert weights, and the
+// workspace of calls streamed under them.
+constexpr FfnSplits kNoPartialTiles = {/*tiled=*/false, /*gateup=*/true};
+
+// A size that only the rule for 1 GB of expert weights takes to the tiled schedule. Its need then differs from the
+// streaming one, either way (74.4 MB tiled and 7.3 MB streamed at T = 432, H = 2048, E = 64, K = 6, I = 1408; 61.3 MB
+// and 75.7 MB at T = 264, H = 4096, E = 8, K = 2, I = 14336), while its neighbours below the line stream.
+bool tiled_by_weight_bytes(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I) {
+    return ffn_schedule(T, H, E, K, I) == 1 && ffn_schedule(T, H, E, K, I, kNoPartialTiles) == 0;
+}
+
+size_t need_bytes(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, FfnSplits splits, bool layer) {
+    return layer ? layer_workspace_bytes(T, H, E, K, I, splits) : ffn_workspace_bytes(T, H, E, K, I, splits);
+}
+
+}  // namespace
+
+// A workspace that holds what streaming needs, but not the tiled schedule's regions, is enough for such a size (it may
+// have been sized for another T): the call streams. Every other size needs its whole workspace.
+FfnSplits workspace_splits(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, size_t bytes, bool layer) {
+    if (bytes < need_bytes(T, H, E, K, I, {}, layer) && tiled_by_weight_bytes(T, H, E, K, I) &&
+        bytes >= need_bytes(T, H, E, K, I, kNoPartialTiles, layer))
+        return kNoPartialTiles;
+    return {};
+}
+
+// The larger of the two needs there, so that a workspace sized for such a T also holds the smaller T that stream.
+size_t workspace_query(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, bool layer) {
+    const size_t need = need_bytes(T, H, E, K, I, {}, layer);
+    if (!tiled_by_weight_bytes(T, H, E, K, I)) return need;
+    const size_t streamed = need_bytes(T, H, E, K, I, kNoPartialTiles, layer);
+    return need > streamed ? need : streamed;
+}
+
 FfnGrid ffn_grid(int T, int H, int E, int K, int I) {
     FfnGrid g;
     g.schedule = ffn_schedule(T, H, E, K, I);
@@ -184,21 +220,22 @@ hipError_t launch_ffn(const uint16_t* x, const int32_t* expert_ids, const uint16
 
 hipError_t launch_ffn_combine(const uint16_t* x, const int32_t* expert_ids, const uint16_t* weights,
                               const uint16_t* expert_weights, uint16_t* expert_out, uint16_t* y, FfnWorkspace ws,
-                              int T, int H, int E, int K, int I, hipStream_t stream) {
-    if (ffn_schedule(T, H, E, K, I) == 0) {
+                              int T, int H, int E, int K, int I, hipStream_t stream, FfnSplits splits) {
+    if (ffn_schedule(T, H, E, K, I, splits) == 0) {
         const hipError_t err = prepare_ffn_stream(H, I);
         if (err != hipSuccess) return err;
-        return launch_ffn_stream(x, expert_ids, expert_weights, expert_out, ws, T, H, E, K, I, stream, weights, y);
+        return launch_ffn_stream(x, expert_ids, expert_weights, expert_out, ws, T, H, E, K, I, stream, weights, y,
+                                 splits.gateup);
     }
-    const hipError_t err = launch_ffn(x, expert_ids, expert_weights, expert_out, ws, T, H, E, K, I, stream);
+    const hipError_t err = launch_ffn(x, expert_ids, expert_weights, expert_out, ws, T, H, E, K, I, stream, splits);
     if (err != hipSuccess) return err;
     return launch_combine(expert_out, weights, y, T, H, K, stream);
 }
 
-size_t layer_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I) {
-    size_t bytes = ffn_workspace_bytes(T, H, E, K, I);
+size_t layer_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, FfnSplits splits) {
+    size_t bytes = ffn_workspace_bytes(T, H, E, K, I, splits);
     // counts for the routing blocks of any routing kernel: at most one block per 16 tokens
-    if (ffn_schedule(T, H, E, K, I) == 1)
+    if (ffn_schedule(T, H, E, K, I, splits) == 1)
         bytes += align_up(sizeof(int32_t) * static_cast<size_t>((T + 15) / 16) * counts_stride(static_cast<int>(E)), 256);
     else  // the split routing's quarter sums (small batches, E > 64)
         bytes += align_up(routing_split_workspace_bytes(static_cast<int>(T), static_cast<int>(E)), 256);
@@ -207,15 +244,16 @@ size_t layer_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t K, int64_t
 
 hipError_t launch_layer(const uint16_t* x, const uint16_t* w_gate, const uint16_t* expert_weights, int32_t* ids,
                         uint16_t* weights, uint16_t* expert_out, uint16_t* y, void* workspace, int T, int H, int E,
-                        int K, int I, hipStream_t stream) {
-    const FfnWorkspace ws = ffn_workspace_carve(workspace, T, H, E, K, I);
-    switch (ffn_schedule(T, H, E, K, I)) {
+                        int K, int I, hipStream_t stream, FfnSplits splits) {
+    const FfnWorkspace ws = ffn_workspace_carve(workspace, T, H, E, K, I, splits);
+    // what follows the FFN's regions: the routing blocks' counts (tiled) or the split routing's sums (streaming)
+    char* const tail = static_cast<char*>(workspace) + ffn_workspace_bytes(T, H, E, K, I, splits);
+    switch (ffn_schedule(T, H, E, K, I, splits)) {
         case 1: {
             hipError_t err = prepare_ffn_tiled();
             if (err != hipSuccess) return err;
-            // rank [T*K] in the permute's scratch; the routing blocks' counts after the FFN workspace
-            int32_t* rank = ws.pscratch;
-            int32_t* counts = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + ffn_workspace_bytes(T, H, E, K, I));
+            int32_t* rank = ws.pscratch;  // [T*K] in the permute's scratch
+            int32_t* counts = reinterpret_cast<int32_t*>(tail);
             err = launch_routing_topk(x, w_gate, ids, weights, T, H, E, K, stream, counts, rank);
             if (err != hipSuccess) return err;
             const bool lw = routing_lds_weights(w_gate, H, E);  // the same choice the routing launch makes
@@ -223,7 +261,7 @@ hipError_t launch_layer(const uint16_t* x, const uint16_t* w_gate, const uint16_
             err = launch_permute_scatter(ids, T * K, E, H, counts, rank, nblocks, routing_tokens_per_block(T, H, E, lw) * K,
                                          permute_scatter_chunks_per_block(nblocks), ws, expert_out, stream);
             if (err != hipSuccess) return err;
-            err = launch_ffn_tiled(x, expert_weights, expert_out, ws, T, H, E, K, I, stream, /*allow_split=*/true);
+            err = launch_ffn_tiled(x, expert_weights, expert_out, ws, T, H, E, K, I, stream, splits.tiled);
             if (err != hipSuccess) return err;
             return launch_combine(expert_out, weights, y, T, H, K, stream);
         }
@@ -231,13 +269,12 @@ hipError_t launch_layer(const uint16_t* x, const uint16_t* w_gate, const uint16_
             hipError_t err = prepare_ffn_stream(H, I);  // the FFN kernels' attributes before the first launch
             if (err != hipSuccess) return err;
             if (routing_split_applies(T, H, E, routing_lds_weights(w_gate, H, E))) {
-                float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + ffn_workspace_bytes(T, H, E, K, I));
-                err = launch_routing_split(x, w_gate, ids, weights, T, H, E, K, part, stream);
+                err = launch_routing_split(x, w_gate, ids, weights, T, H, E, K, reinterpret_cast<float*>(tail), stream);
             } else {
                 err = launch_routing_topk(x, w_gate, ids, weights, T, H, E, K, stream);
             }
             if (err != hipSuccess) return err;
-            return launch_ffn_combine(x, ids, weights, expert_weights, expert_out, y, ws, T, H, E, K, I, stream);
+            return launch_ffn_combine(x, ids, weights, expert_weights, expert_out, y, ws, T, H, E, K, I, stream, splits);
         }
         default: return hipErrorInvalidValue;
     }

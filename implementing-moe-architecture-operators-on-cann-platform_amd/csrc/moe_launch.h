@@ -71,7 +71,11 @@ struct FfnSplits {
 };
 size_t ffn_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, FfnSplits splits = {});
 FfnWorkspace ffn_workspace_carve(void* base, int64_t T, int64_t H, int64_t E, int64_t K, int64_t I,
-                                 FfnSplits splits = {});
+                                 FfnSplits splits);
+// The splits of a call whose caller gave `bytes` of workspace (layer: of moe_layer, else of the FFN)
+FfnSplits workspace_splits(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, size_t bytes, bool layer);
+// The workspace a caller is told to give
+size_t workspace_query(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, bool layer);
 
 int permute_block_threads();
 int permute_chunks(int S);
@@ -136,21 +140,21 @@ int ffn_schedule(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, FfnSplit
 // kernel's attributes are set before the first launch, so a failure there leaves nothing launched.
 hipError_t launch_ffn(const uint16_t* x, const int32_t* expert_ids, const uint16_t* expert_weights,
                       uint16_t* expert_out, FfnWorkspace ws, int T, int H, int E, int K, int I, hipStream_t stream,
-                      FfnSplits splits = {});
+                      FfnSplits splits);
 // the FFN followed by the combine: expert_out as launch_ffn writes it, y as launch_combine would compute it
 hipError_t launch_ffn_combine(const uint16_t* x, const int32_t* expert_ids, const uint16_t* weights,
                               const uint16_t* expert_weights, uint16_t* expert_out, uint16_t* y, FfnWorkspace ws,
-                              int T, int H, int E, int K, int I, hipStream_t stream);
+                              int T, int H, int E, int K, int I, hipStream_t stream, FfnSplits splits);
 
 // ---- the whole layer: routing -> FFN -> combine in one call (moe_ffn.hip) ----
 // workspace: the FFN's (ffn_workspace_bytes), then on the tiled schedule the routing blocks' expert counts
-size_t layer_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I);
+size_t layer_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, FfnSplits splits = {});
 // Tiled schedule: the routing kernel also ranks its blocks' slots (the permute's count), then one scatter launch,
 // the two GEMMs and the combine. Streaming schedule: routing, then launch_ffn_combine. ids, weights, expert_out
 // and y equal the three operators' bit for bit.
 hipError_t launch_layer(const uint16_t* x, const uint16_t* w_gate, const uint16_t* expert_weights, int32_t* ids,
                         uint16_t* weights, uint16_t* expert_out, uint16_t* y, void* workspace, int T, int H, int E,
-                        int K, int I, hipStream_t stream);
+                        int K, int I, hipStream_t stream, FfnSplits splits);
 
 // ---- fixed scratch of the allocation-free FFN entry point (moe_noalloc.hip) ----
 size_t noalloc_scratch_bytes();

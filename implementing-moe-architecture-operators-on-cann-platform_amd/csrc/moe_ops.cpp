@@ -220,7 +220,7 @@ moe_status moe_expert_ffn_infer_dtype(moe_dtype* expert_out_dtype) {
 
 size_t moe_expert_ffn_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I) {
     if (check_ffn_sizes(T, H, E, K, I) != MOE_OK) return 0;
-    return moe::ffn_workspace_bytes(T, H, E, K, I);
+    return moe::workspace_query(T, H, E, K, I, /*layer=*/false);
 }
 
 moe_status moe_expert_ffn_plan(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, moe_ffn_plan* plan) {
@@ -240,7 +240,7 @@ moe_status moe_expert_ffn_plan(int64_t T, int64_t H, int64_t E, int64_t K, int64
     plan->down_grid = g.down_blocks;
     plan->block = g.block_threads;
     plan->rows_per_tile = g.rows_per_tile;
-    plan->workspace_bytes = moe::ffn_workspace_bytes(T, H, E, K, I);
+    plan->workspace_bytes = moe::workspace_query(T, H, E, K, I, /*layer=*/false);
     return ok();
 }
 
@@ -254,17 +254,18 @@ moe_status moe_expert_ffn(const uint16_t* x, const int32_t* expert_ids, const ui
     if (T == 0) return ok();
     if (!x || !expert_ids || !expert_weights || !expert_out)
         return fail(MOE_ERR_NULL, "MoeExpertFFN: null tensor pointer");
-    const size_t need = moe::ffn_workspace_bytes(T, H, E, K, I);
+    const moe::FfnSplits splits = moe::workspace_splits(T, H, E, K, I, workspace_bytes, /*layer=*/false);
+    const size_t need = moe::ffn_workspace_bytes(T, H, E, K, I, splits);
     if (!workspace || workspace_bytes < need)
         return fail(MOE_ERR_WORKSPACE, "MoeExpertFFN: workspace %zu bytes at %p, need %zu", workspace_bytes,
                     workspace, need);
     if (!aligned16(x) || !aligned16(expert_weights) || !aligned16(expert_out) || !aligned16(workspace))
         return fail(MOE_ERR_UNSUPPORTED, "MoeExpertFFN: x, expert_weights, expert_out, workspace must be 16-byte aligned");
     const hipStream_t s = as_stream(stream);
-    const moe::FfnWorkspace ws = moe::ffn_workspace_carve(workspace, T, H, E, K, I);
+    const moe::FfnWorkspace ws = moe::ffn_workspace_carve(workspace, T, H, E, K, I, splits);
     const hipError_t err = moe::launch_ffn(x, expert_ids, expert_weights, expert_out, ws, static_cast<int>(T),
                                            static_cast<int>(H), static_cast<int>(E), static_cast<int>(K),
-                                           static_cast<int>(I), s);
+                                           static_cast<int>(I), s, splits);
     if (err != hipSuccess) return hip_fail(err, "MoeExpertFFN GEMM launch");
     return ok();
 }
@@ -323,7 +324,8 @@ moe_status moe_expert_ffn_combine(const uint16_t* x, const int32_t* expert_ids, 
     if (T == 0) return ok();
     if (!x || !expert_ids || !weights || !expert_weights || !expert_out || !y)
         return fail(MOE_ERR_NULL, "MoeExpertFFN+MoeCombine: null tensor pointer");
-    const size_t need = moe::ffn_workspace_bytes(T, H, E, K, I);
+    const moe::FfnSplits splits = moe::workspace_splits(T, H, E, K, I, workspace_bytes, /*layer=*/false);
+    const size_t need = moe::ffn_workspace_bytes(T, H, E, K, I, splits);
     if (!workspace || workspace_bytes < need)
         return fail(MOE_ERR_WORKSPACE, "MoeExpertFFN+MoeCombine: workspace %zu bytes at %p, need %zu", workspace_bytes,
                     workspace, need);
@@ -332,10 +334,10 @@ moe_status moe_expert_ffn_combine(const uint16_t* x, const int32_t* expert_ids, 
         return fail(MOE_ERR_UNSUPPORTED,
                     "MoeExpertFFN+MoeCombine: x, expert_weights, expert_out, y, workspace must be 16-byte aligned");
     const hipStream_t s = as_stream(stream);
-    const moe::FfnWorkspace ws = moe::ffn_workspace_carve(workspace, T, H, E, K, I);
+    const moe::FfnWorkspace ws = moe::ffn_workspace_carve(workspace, T, H, E, K, I, splits);
     const hipError_t err = moe::launch_ffn_combine(x, expert_ids, weights, expert_weights, expert_out, y, ws,
                                                    static_cast<int>(T), static_cast<int>(H), static_cast<int>(E),
-                                                   static_cast<int>(K), static_cast<int>(I), s);
+                                                   static_cast<int>(K), static_cast<int>(I), s, splits);
     if (err != hipSuccess) return hip_fail(err, "MoeExpertFFN+MoeCombine launch");
     return ok();
 }
@@ -343,7 +345,7 @@ moe_status moe_expert_ffn_combine(const uint16_t* x, const int32_t* expert_ids, 
 // The whole layer in one call (optional fast path; the three operators stay the contract)
 size_t moe_layer_workspace_bytes(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I) {
     if (check_ffn_sizes(T, H, E, K, I) != MOE_OK) return 0;
-    return moe::layer_workspace_bytes(T, H, E, K, I);
+    return moe::workspace_query(T, H, E, K, I, /*layer=*/true);
 }
 
 moe_status moe_layer(const uint16_t* x, const uint16_t* w_gate, const uint16_t* expert_weights, int32_t* expert_ids,
@@ -356,7 +358,8 @@ moe_status moe_layer(const uint16_t* x, const uint16_t* w_gate, const uint16_t* 
     if (T == 0) return ok();
     if (!x || !w_gate || !expert_weights || !expert_ids || !weights || !expert_out || !y)
         return fail(MOE_ERR_NULL, "MoE layer: null tensor pointer");
-    const size_t need = moe::layer_workspace_bytes(T, H, E, K, I);
+    const moe::FfnSplits splits = moe::workspace_splits(T, H, E, K, I, workspace_bytes, /*layer=*/true);
+    const size_t need = moe::layer_workspace_bytes(T, H, E, K, I, splits);
     if (!workspace || workspace_bytes < need)
         return fail(MOE_ERR_WORKSPACE, "MoE layer: workspace %zu bytes at %p, need %zu", workspace_bytes, workspace,
                     need);
@@ -365,7 +368,7 @@ moe_status moe_layer(const uint16_t* x, const uint16_t* w_gate, const uint16_t* 
         return fail(MOE_ERR_UNSUPPORTED, "MoE layer: x, expert_weights, expert_out, y, workspace must be 16-byte aligned");
     const hipError_t err = moe::launch_layer(x, w_gate, expert_weights, expert_ids, weights, expert_out, y, workspace,
                                              static_cast<int>(T), static_cast<int>(H), static_cast<int>(E),
-                                             static_cast<int>(K), static_cast<int>(I), as_stream(stream));
+                                             static_cast<int>(K), static_cast<int>(I), as_stream(stream), splits);
     if (err != hipSuccess) return hip_fail(err, "MoE layer launch");
     return ok();
 }

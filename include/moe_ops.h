@@ -126,7 +126,11 @@ moe_status moe_expert_ffn_infer_dtype(moe_dtype* expert_out_dtype);
  * slot order, per-expert offsets and the fp16 SwiGLU intermediate [T*K, I]; on the weight-streaming schedule
  * also the split-K partial sums and the slot -> sorted-row map; on the LDS-tiled schedule also up to 64 MiB of
  * fp32 partial tiles for the tiles it splits over k (only when its down tiles fill at most 4 rounds of the
- * GPU). 0 for invalid sizes. */
+ * GPU). 0 for invalid sizes.
+ * Not monotone in num_tokens: a caller that keeps one workspace over its calls takes the largest over every
+ * num_tokens it will use. Where the expert weights reach 1 GB and only that takes a size to the tiled schedule, the
+ * value covers both schedules, and a call given less than the tiled schedule needs, but enough to stream, streams:
+ * its expert_out then differs from that of a call with the whole workspace in fp32 summation order. */
 size_t moe_expert_ffn_workspace_bytes(int64_t num_tokens, int64_t hidden_size, int64_t num_experts,
                                       int64_t top_k, int64_t intermediate_size);
 
@@ -223,8 +227,10 @@ moe_status moe_expert_ffn_combine(const uint16_t* x, const int32_t* expert_ids, 
  * scatter launch after it (the per-expert id scan of op_kernel/moe_expert_ffn.cpp:182-195, done once); on the
  * weight-streaming schedule it is routing (for T <= 16 and E > 64 spread over 4 * E / 32 workgroups, whose fp32
  * sums pass through the workspace) followed by moe_expert_ffn_combine. expert_ids, weights, expert_out and y are
- * bit-identical to the three calls'. Deterministic (no global atomics; nothing depends on timing).
- * The workspace is moe_layer_workspace_bytes() (>= moe_expert_ffn_workspace_bytes()); 0 = unsupported sizes.
+ * bit-identical to the three calls' (each with the workspace of its own query). Deterministic (no global atomics;
+ * nothing depends on timing).
+ * The workspace is moe_layer_workspace_bytes() (>= moe_expert_ffn_workspace_bytes()); 0 = unsupported sizes; not
+ * monotone in num_tokens and covering both schedules, as moe_expert_ffn_workspace_bytes().
  * Sizes and errors as the three operators' checks together.
  * ---------------------------------------------------------------------------------------------------- */
 size_t moe_layer_workspace_bytes(int64_t num_tokens, int64_t hidden_size, int64_t num_experts, int64_t top_k,

@@ -366,3 +366,39 @@ def test_fused_layer_takes_as_many_experts_as_it_routes_to(monkeypatch):
         assert not calls
     ops.moe_layer_fused(x, torch.zeros((64, 8), dtype=torch.float16), ew, 2)
     assert len(calls) == 1
+
+
+@pytest.mark.parametrize("H,E,K,I,kept,sizes", [
+    (2048, 64, 6, 1408, 2736, range(427, 761)),  # kept: tiled, no partial tiles; sizes: tiled from 1 GB of weights
+    (4096, 8, 2, 14336, 264, range(1, 264)),     # kept: tiled from 1 GB of weights; sizes: streamed
+])
+def test_kept_workspace_covers_the_sizes_it_covered(lib, H, E, K, I, kept, sizes):
+    """The workspace need is not monotone in T: split partial sums and up to 64 MiB of partial tiles come and go. Where
+    the expert weights reach 1 GB the tiled schedule takes over earlier, and a workspace sized for one T stays enough
+    for the T it was enough for without that: the query gives the larger of the two schedules' needs, and a call whose
+    workspace holds the streaming need only streams. Each call gets past the workspace check (to the alignment check,
+    on an x of odd address; nothing is launched). One byte under the smaller need, and one byte under the need of a
+    size that is tiled either way, are refused."""
+    odd, ok = 0x10001, 0x10000
+
+    def ffn(T, nbytes):
+        return lib.moe_expert_ffn(odd, ok, ok, ok, ok, ok, nbytes, T, H, E, K, I, None)
+
+    def ffn_combine(T, nbytes):
+        return lib.moe_expert_ffn_combine(odd, ok, ok, ok, ok, ok, ok, nbytes, T, H, E, K, I, None)
+
+    def layer(T, nbytes):
+        return lib.moe_layer(odd, ok, ok, ok, ok, ok, ok, ok, nbytes, T, H, E, K, I, None)
+
+    for call, query in [(ffn, lib.moe_expert_ffn_workspace_bytes), (ffn_combine, lib.moe_expert_ffn_workspace_bytes),
+                        (layer, lib.moe_layer_workspace_bytes)]:
+        nbytes = query(kept, H, E, K, I)
+        for T in sizes:
+            assert call(T, nbytes) == ERR_UNSUP, (T, lib.moe_last_error())
+            assert b"16-byte aligned" in lib.moe_last_error()
+        T = sizes[0]
+        least = next(n for n in range(2 * T * K * I, nbytes + 1, 256) if call(T, n) != ERR_WS)
+        assert call(T, least - 1) == ERR_WS
+        T = 100 * E // K  # 100 rows per expert: tiled under every line
+        assert call(T, query(T, H, E, K, I) - 1) == ERR_WS
+        assert call(T, query(T, H, E, K, I)) == ERR_UNSUP

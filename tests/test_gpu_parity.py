@@ -1474,3 +1474,38 @@ def test_permute_slot_counts(ops, S, E):
     eo_d, ws = run_ffn(ops, dev(x), dev(ids), dev(w), dev(ew), I)
     check_permute(host(ws), ids, E)
     assert not host(eo_d)[bad].any()
+
+
+def test_kept_workspace_streams_where_tiled_does_not_fit(ops):
+    """1.1 GB of expert weights at 40.5 rows per expert: tiled, with 64 MiB of partial tiles in its workspace. Given
+    only the bytes that streaming needs (a workspace kept from another batch size) the FFN, FFN + combine and moe_layer
+    calls stream, agree bit for bit, leave the bytes behind the workspace alone and match the oracle on 16 tokens; the
+    whole workspace gives the same rows up to the fp16 rounding of hidden and of the result (2^-11 each of values below
+    8, twice)."""
+    T, H, E, K, I = 432, 2048, 64, 6, 1408
+    assert ffn_schedule(T, H, E, K, I) == 1
+    lib = ops._lib.load()
+    # the least workspace that passes the size check: the call then fails on x's odd address, nothing is launched
+    least = next(n for n in range(2 * T * K * I, 1 << 24, 256)
+                 if lib.moe_expert_ffn(0x10001, 0x10000, 0x10000, 0x10000, 0x10000, 0x10000, n, T, H, E, K, I, None) == 6)
+    log(f"[kept workspace] streaming need {least} bytes, query {ops.workspace_bytes(T, H, E, K, I)}")
+    x = torch.empty((T, H), dtype=torch.float16, device="cuda")
+    ops.synth_normal_f16_(x, 23, synth.STREAM_X, 1.0)
+    ew = torch.empty((E, 3 * I, H), dtype=torch.float16, device="cuda")
+    ops.synth_normal_f16_(ew, 23, synth.STREAM_EXPERT_WEIGHTS, 1.0 / math.sqrt(H), 1.0 / math.sqrt(I), 3 * I * H,
+                          2 * I * H)
+    rng = np.random.default_rng(23)
+    wg = dev((rng.standard_normal((H, E)) / math.sqrt(H)).astype(np.float16))
+    buf = torch.full((least + 4096,), 0xA5, dtype=torch.uint8, device="cuda")
+    y, ids, w, eo = ops.moe_layer(x, wg, ew, K, buf[:least])
+    eo_c, y_c = ops.MoeExpertFFNCombine(x, ids, w, ew, 0, buf[:least])
+    y_f, ids_f, w_f, eo_f = ops.moe_layer_fused(x, wg, ew, K, 0, buf[:least])
+    for a, b in ((eo, eo_c), (y, y_c), (eo, eo_f), (y, y_f), (ids, ids_f), (w, w_f)):
+        assert torch.equal(a, b)
+    assert (buf[least:] == 0xA5).all()
+    eo_h, ids_h = f32(host(eo)), host(ids)
+    n = 16
+    within(oracle.compare(eo_h[:n], oracle_ffn_threads(f32(host(x))[:n], ids_h[:n], f32(host(ew)), I)), max_abs=1e-2,
+           mean_abs=1e-3, cos=0.9999)
+    full = f32(host(ops.moe_layer(x, wg, ew, K)[3]))
+    within(oracle.compare(eo_h, full), max_abs=2**-6, mean_abs=2**-10, cos=0.9999)
