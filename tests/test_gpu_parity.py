@@ -1509,3 +1509,46 @@ def test_kept_workspace_streams_where_tiled_does_not_fit(ops):
            mean_abs=1e-3, cos=0.9999)
     full = f32(host(ops.moe_layer(x, wg, ew, K)[3]))
     within(oracle.compare(eo_h, full), max_abs=2**-6, mean_abs=2**-10, cos=0.9999)
+
+
+@pytest.mark.parametrize("H,I,E,gemm", [
+    # gate/up: reductions of 2, 3 and 5 stages, ending in a half stage (odd multiple of 32) and whole
+    (96, 2048, 40, "gateup"), (128, 2048, 40, "gateup"), (160, 2048, 40, "gateup"), (192, 2048, 40, "gateup"),
+    (288, 2048, 40, "gateup"), (320, 2048, 40, "gateup"),
+    # down: the same reductions; with E = 20 its leftover round is split over k as well
+    (4096, 96, 40, "down"), (4096, 128, 40, "down"), (4096, 160, 40, "down"), (4096, 192, 40, "down"),
+    (4096, 288, 40, "down"), (4096, 320, 40, "down"), (4096, 288, 20, "down"), (4096, 320, 20, "down"),
+])
+def test_tiled_short_reductions_over_several_tiles(ops, H, I, E, gemm):
+    """Workgroups of the tiled kernels that go on to further tiles while a tile has few stages: below 4 the next tile's
+    plan is made after a full wait, at 2 between the two halves of its first stage, and a half stage is followed by the
+    next tile's. More tiles than workgroups in the named GEMM, ragged m-tiles, an expert without rows; two runs agree
+    bit for bit, and the rows around every 64-row and 256-row edge of every expert match the oracle. Bounds as in
+    test_tiled_tile_and_stage_edges."""
+    edges = [1, 127, 128, 129, 255, 256, 257, 64, 0, 385, 513, 192]
+    rows = [edges[e % len(edges)] for e in range(E)]
+    T = sum(rows)
+    tiles = sum(-(-r // 256) for r in rows) * (-(-I // 128) if gemm == "gateup" else -(-H // 256))
+    assert tiles > torch.cuda.get_device_properties(0).multi_processor_count
+    assert ffn_schedule(T, H, E, 1, I) == 1
+    rng = np.random.default_rng(H * 1000 + I + E)
+    ids = rng.permutation(np.repeat(np.arange(E, dtype=np.int32), rows)).reshape(T, 1)
+    x = rng.standard_normal((T, H), dtype=np.float32).astype(np.float16)
+    ew = np.concatenate([rng.standard_normal((E, 2 * I, H), dtype=np.float32) / math.sqrt(H),
+                         rng.standard_normal((E, I, H), dtype=np.float32) / math.sqrt(I)], axis=1).astype(np.float16)
+    x_d, ids_d, w_d, ew_d = dev(x), dev(ids), dev(np.ones((T, 1), np.float16)), dev(ew)
+    with ops.kernel_trace() as launched:
+        eo_d = ops.MoeExpertFFN(x_d, ids_d, w_d, ew_d)
+        torch.cuda.synchronize()
+    log(f"[short reductions] H={H} I={I} E={E}: {tiles} {gemm} tiles, kernels {sorted(launched)}")
+    assert gemm == "gateup" or ("moe_ffn_down_fixup" in launched) == (E == 20)
+    assert torch.equal(eo_d, ops.MoeExpertFFN(x_d, ids_d, w_d, ew_d))
+    tok = []
+    for e in range(E):
+        own = np.nonzero(ids[:, 0] == e)[0]  # the expert's rows in sorted order
+        at = {p + d for p in range(0, len(own) + 1, 64) for d in (-1, 0)} | {len(own) - 1}
+        tok += [own[p] for p in sorted(at) if 0 <= p < len(own)]
+    tok = np.array(tok)
+    eo = f32(host(eo_d))[tok]
+    within(oracle.compare(eo, oracle_ffn_threads(f32(x[tok]), ids[tok], f32(ew), I)), max_abs=2**-6, mean_abs=2**-10,
+           cos=0.9999)
