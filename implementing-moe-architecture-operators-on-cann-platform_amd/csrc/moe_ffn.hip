@@ -23,44 +23,43 @@ size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // Average rows per expert from which the tiled schedule runs. The 32-row streaming kernels stream every expert's
 // weights once per 32 rows, so they degrade once experts exceed 32 rows; the wide streaming kernels take up to 128
-// rows per pass and run in their place from 32 rows (moe_ffn_stream.hip); the tiled kernels cost about the same
-// from 32 to 256 rows (their 256-row tiles are then mostly padding). H = 2048, E = 16, K = 2, I = 8192, the FFN's
-// kernels on one box (32-row streaming / wide streaming / tiled):
-//   T = 128 (16 rows per expert)   273 / -   / 466 us
-//   T = 256 (32)                    451 / 364 / 449-493 us
-//   T = 384 (48)                    541 / 385 / 458-491 us
-//   T = 512 (64)                    707 / 440 / 452-477 us
-//   T = 768 (96)                      - / 496 / 465-482 us
-//   T = 1024 (128)                 1271 / 734 / 480-491 us
-// The wide/tiled crossover moves with I: the FFN (wide / tiled, us) at 64 and 80 rows per expert on average:
-//   H = 2048, E = 16, K = 2, I = 8192     420 / 501,  445 / 496   (wide still ahead at 80 rows)
-//   H = 4096, E = 8,  K = 2, I = 14336    676 / 816,  765 / 843
-//   H = 2048, E = 64, K = 6, I = 1408     332 / 353,  350 / 333   (crossover ~72 rows)
-//   H = 4096, E = 128, K = 8, I = 1536   1160 / 1241, 1264 / 1250  (~77)
-//   H = 5120, E = 16, K = 2, I = 1536     241 / 253,  270 / 264   (~74)
-//   H = 7168, E = 256, K = 8, I = 2048   5427 / 5297 at 64 rows, 5029 / 5259 at 56  (~61)
-// so the wide kernels run to 72 rows below I = 4096. From I = 4096 they run to 96 rows, measured again with the
-// wide kernels' short passes (moe_ffn_stream.hip), the FFN (wide / tiled, us, one box):
-//   H = 2048, E = 16, K = 2, I = 8192     80 rows 408.6 / 442.2, 88 rows 419.6 / 452.4, 96 rows 431.8 / 450.8,
-//                                         112 rows 612.5 / 468.1 (experts above 128 rows take a second pass)
-//   H = 4096, E = 8,  K = 2, I = 14336    80 rows 726.7 / 784.0, 96 rows 779.1 / 804.8, 112 rows 1143.3 / 822.5
-// Shapes the wide kernels cannot run switch to the tiled schedule at 32 rows.
-// Expert weights of at least 1 GB (streamed from HBM whichever schedule runs, for long enough that the tiled one's
-// permute and fix-up launches do not show) switch earlier: the tiled kernels then cost the same from ~32 to ~100 rows
-// per expert, and with many or unevenly loaded experts the wide kernels' time is that of the fullest ones. The FFN
-// (wide / tiled, us, one box; Zipf = Zipf-skewed routing):
-//   H = 2048, E = 16, K = 2, I = 8192     56 rows 357.1 / 363.8, 64 rows 358.9 / 362.3, 72 rows 383.7 / 373.1,
-//                                         96 rows 427.6 / 373.1
-//   H = 4096, E = 8,  K = 2, I = 14336    40 rows 561.2 / 601.3, 56 rows 637.2 / 618.3, 72 rows 684.1 / 620.1
-//   H = 2048, E = 64, K = 6, I = 1408     32 rows 236.8 / 236.4, 40 rows 243.8 / 234.3, 56 rows 266.5 / 239.1
-//   H = 4096, E = 128, K = 8, I = 1536    40 rows 905.5 / 889.5, 56 rows 1043.4 / 923.9, 70 rows 1143.0 / 947.2
-//   H = 7168, E = 256, K = 8, I = 2048    37 rows 4156.6 / 4165.7, 60 rows 5365.6 / 4348.2
-//   H = 1024, E = 64, K = 4, I = 3072     37 rows 254.5 / 258.5, 50 rows 284.5 / 263.7
-//   Zipf: H = 2048, E = 16, I = 8192 72 rows 758.6 / 431.0; H = 2048, E = 64, I = 1408 37 rows 482.4 / 237.6
-// Below 1 GB the lines above hold (H = 1024, E = 96, K = 4, I = 1024: 40 rows 146.8 / 181.3; H = 1536, E = 12, K = 2,
-// I = 6144: 66 rows 203.1 / 231.6; H = 1024, E = 32, K = 4, I = 4096: 65 rows 197.7 / 205.1). Calls
-// without the split leftover round's workspace (splits.tiled off) and sizes past the tiled kernels' offsets keep them
-// too.
+// rows per pass and run in their place from 32 rows at the latest (moe_ffn_stream.hip); the tiled kernels cost about
+// the same from 32 to ~110 rows per expert (their 256-row tiles are then mostly padding). The host sees only the
+// average: the wide kernels' time is that of the fullest experts, so it grows with uneven loads, the tiled kernels'
+// hardly. The FFN alone, ids drawn uniformly (wide / tiled, us, one box):
+//   H = 2048, E = 16, K = 2, I = 8192   32 rows 305 / 362, 48 rows 323 / 360, 56 rows 370 / 363, 64 rows 376 / 362,
+//     (1.6 GB)                          72 rows 397 / 369, 96 rows 452 / 375, 112 rows 484 / 384, 128 rows 699 / 394
+//   H = 4096, E = 8, K = 2, I = 14336   40 rows 559 / 599, 56 rows 597 / 612, 64 rows 664 / 622, 72 rows 707 / 624,
+//     (2.8 GB)                          96 rows 794 / 641, 112 rows 839 / 657
+//   H = 2048, E = 64, K = 6, I = 1408   32 rows 241 / 236, 40 rows 248 / 233, 56 rows 280 / 239, 72 rows 304 / 246
+//     (1.1 GB)
+//   H = 4096, E = 128, K = 8, I = 1536  32 rows 868 / 900, 40 rows 915 / 911, 56 rows 1059 / 942, 70 rows 1161 / 951
+//   H = 7168, E = 256, K = 8, I = 2048  37 rows 4001 / 4202, 48 rows 4788 / 4300, 64 rows 5339 / 4397
+//   H = 1024, E = 64, K = 4, I = 3072   32 rows 253 / 255, 40 rows 265 / 257, 64 rows 308 / 266  (1.2 GB)
+//   H = 5120, E = 16, K = 2, I = 1536   40 rows 185 / 202, 56 rows 213 / 206, 72 rows 237 / 205  (0.75 GB)
+//   H = 1024, E = 96, K = 4, I = 1024   40 rows 144 / 174, 64 rows 177 / 181, 72 rows 200 / 184  (0.6 GB)
+//   H = 2048, E = 32, K = 4, I = 1408   48 rows 157 / 158, 64 rows 168 / 161, 72 rows 179 / 162  (0.55 GB)
+//   H = 1536, E = 12, K = 2, I = 6144   66 rows 198 / 219, 80 rows 215 / 220, 96 rows 228 / 225, 104 rows 235 / 229
+//     (0.7 GB)
+//   H = 1024, E = 32, K = 4, I = 4096   48 rows 194 / 202, 56 rows 208 / 204, 65 rows 215 / 205, 80 rows 238 / 211,
+//     (0.8 GB)                          96 rows 255 / 215
+//   Zipf-skewed ids: H = 2048, E = 16, I = 8192 56 rows 940 / 425, 96 rows 1665 / 455; H = 2048, E = 64, I = 1408
+//   32 rows 732 / 256, 64 rows 1373 / 307; H = 1024, E = 32, I = 4096 48 rows 542 / 220, 80 rows 873 / 252
+// Three lines:
+//   32 rows      shapes the wide kernels cannot run.
+//   72 rows, and 97 from I = 4096   expert weights below 1 GB. Both were drawn on a slower tiled kernel: by the table
+//                the present one wins from ~56-68 rows (H = 1536, E = 12 from ~90).
+//   40 rows (E >= 64), 66 rows      expert weights of at least 1 GB, streamed from HBM whichever schedule runs for long
+//                enough that the tiled one's permute and fix-up launches do not show. Calls without the split leftover
+//                round's workspace (splits.tiled off) and sizes past the tiled kernels' offsets keep the lines above.
+// Where the 1 GB line loses on even loads: 1 GB over few down output columns (E * H / 256 tiles) means a long I and few
+// down tiles, each split over k. 64 tiles: H = 1024, E = 16, I = 14336 66 rows 352 / 426, 95 rows 411 / 445; H = 2048,
+// E = 8, I = 14336 66 rows 365 / 420; H = 512, E = 32, I = 14336 66 rows 388 / 451; H = 256, E = 64, I = 14336 40 rows
+// 424 / 477. 80 tiles: H = 2560, E = 8, I = 9216 66 rows 300 / 325, 85 rows 345 / 338. 96 tiles: H = 384, E = 64,
+// I = 12288 40 rows 473 / 504, 52 rows 522 / 507; H = 768, E = 32, I = 8192 66 rows 342 / 329. It holds there all the
+// same, for with a gate of Zipf-scaled columns the same sizes take (wide / tiled) 686 / 487 and 1006 / 492, 391 / 431
+// (80 rows 572 / 448), 1477 / 499, 1256 / 495; H = 1280, E = 16, I = 9216 66 rows 598 / 371; 1412 / 490 at E = 64,
+// H = 384.
 constexpr int64_t kTiledMinRowsPerExpert = 32;
 constexpr int64_t kWideMaxRowsPerExpert = 97;
 constexpr int64_t kWideMaxRowsSmallI = 72;
