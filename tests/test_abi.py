@@ -120,21 +120,21 @@ def test_plans(lib):
     # E <= 32: the narrow kernel at any T (16 waves, up to 4 token blocks a workgroup)
     assert lib.moe_routing_topk_plan(8192, 2048, 16, 2, C.byref(rp)) == MOE_OK
     assert (rp.grid, rp.block, rp.tokens_per_block, rp.lds_bytes) == (256, 1024, 32, 16 * (32 * 16 * 4 + 32 * 16 * 2))
-    # E > 64: 64 tokens per workgroup; the rows kernel (4 waves of 16 tokens over all of H, four 16 KB w_gate
-    # stages, each wave's x ring of 16 + 1 k-steps of 1 KB)
+    # E > 64 and T > 8192: the direct kernel, 64 tokens per workgroup, each of its 4 waves a quarter of H. The LDS
+    # reserved holds the exchange of the sums and the logits (at 64 tokens and E = 256: 64 KB and 65 KB)
     assert lib.moe_routing_topk_plan(16384, 2048, 256, 8, C.byref(rp)) == MOE_OK
     assert (rp.grid, rp.block, rp.tokens_per_block) == (256, 256, 64)
-    assert rp.lds_bytes == 4 * 16384 + 4 * (16 + 1) * 1024  # the rows kernel: 4 w_gate stages, x rings
-    # E > 64 and T <= 8192: 16 tokens per workgroup; the quarters kernel (4 waves, each a quarter of H through two
-    # 16 KB w_gate stages and two 1 KB x stages of its own)
+    assert rp.lds_bytes == 4 * 16384 + 4 * (16 + 1) * 1024 >= 64 * 1024 + 64 * (256 + 4) * 4
+    # E > 128 and T <= 4096, E <= 128 and T <= 8192: 16 tokens per workgroup (the exchange then takes 16 KB, the logits
+    # 16 or 8 KB)
     assert lib.moe_routing_topk_plan(128, 7168, 256, 8, C.byref(rp)) == MOE_OK
     assert (rp.grid, rp.block, rp.tokens_per_block, rp.lds_bytes) == (8, 256, 16, 4 * (2 * 16384 + 2 * 1024))
     assert lib.moe_routing_topk_plan(8192, 2048, 128, 8, C.byref(rp)) == MOE_OK
     assert (rp.grid, rp.block, rp.tokens_per_block, rp.lds_bytes) == (512, 256, 16, 4 * (2 * 16384 + 2 * 2 * 1024))
-    # E % 8 != 0 (no 16-byte w_gate rows): the wide kernel, w_gate transposed through LDS
+    # E % 8 != 0 (w_gate rows not 16-byte aligned): the same kernel with 2-byte aligned loads
     assert lib.moe_routing_topk_plan(16384, 2048, 250, 8, C.byref(rp)) == MOE_OK
     assert (rp.grid, rp.block, rp.tokens_per_block) == (256, 256, 64)
-    assert rp.lds_bytes == 2 * 256 * (2 * 32 + 8) * 2 + 64 * 256 * 4  # 2 stages of 64 h, fp32 logits
+    assert rp.lds_bytes == 2 * 256 * (2 * 32 + 8) * 2 + 64 * 256 * 4 == 136 * 1024
     assert lib.moe_routing_topk_plan(128, 2040, 16, 2, C.byref(rp)) == ERR_UNSUP
     assert lib.moe_routing_topk_plan(128, 2048, 300, 2, C.byref(rp)) == ERR_UNSUP
     fp = lib_mod.FfnPlan()

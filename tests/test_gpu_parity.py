@@ -315,8 +315,8 @@ def test_routing_shapes(ops, T, H, E, K):
 @pytest.mark.parametrize("E,K", [(16, 2), (64, 6), (40, 5)])
 def test_routing_is_batch_invariant(ops, E, K):
     """A token's ids and weights do not depend on the batch it is routed in: 16400 tokens run several token
-    blocks per workgroup (E <= 32) or the rows kernel (32 < E <= 64), their first 1000 alone run the narrow
-    kernel with one block, and the rows agree bit for bit."""
+    blocks per workgroup of the narrow kernel (4 for E <= 32, 2 above), their first 1000 alone one, and the rows agree
+    bit for bit."""
     T, H = 16400, 512
     rng = np.random.default_rng(E)
     x = rng.standard_normal((T, H)).astype(np.float16)
@@ -359,11 +359,10 @@ def test_routing_resident_kernel_matches_narrow(ops, T, H, E, K):
     (160, 256, 4),   # 5 stages: quarters of 1, 1, 1 and 2 stages
     (128, 128, 2),   # 2 stages: quarters 0 and 2 empty
 ])
-def test_routing_quarters_and_rows_kernels_agree(ops, H, E, K):
-    """E > 64: up to 8192 tokens the quarters kernel routes (16 tokens a workgroup, a wave per quarter of H), above
-    that the rows kernel (64 tokens a workgroup, the quarters one after the other in each wave). Both add a token's
-    H in the same four quarter sums, so 8300 tokens routed together and their first 1000 routed alone agree bit for
-    bit; the small batch is also checked against the oracle's routing."""
+def test_routing_direct_kernel_16_and_64_tokens_agree(ops, H, E, K):
+    """E > 64: the direct kernel routes 16 tokens a workgroup in small batches and 64 from 8193 tokens, each of its
+    waves a quarter of H. Both add a token's H in the same four quarter sums, so 8300 tokens routed together and their
+    first 1000 routed alone agree bit for bit; the small batch is also checked against the oracle's routing."""
     T = 8300
     rng = np.random.default_rng(H + E)
     x = rng.standard_normal((T, H)).astype(np.float16)
@@ -373,16 +372,16 @@ def test_routing_quarters_and_rows_kernels_agree(ops, H, E, K):
     ids_few, w_few = host(ids_few), host(w_few)
     assert np.array_equal(host(ids_all)[:1000], ids_few)
     assert np.array_equal(host(w_all)[:1000].view(np.uint16), w_few.view(np.uint16))
-    check_routing(ids_few, w_few, x[:1000], wg, K, f"quarters H{H} E{E} K{K}")
+    check_routing(ids_few, w_few, x[:1000], wg, K, f"direct H{H} E{E} K{K}")
 
 
-def test_routing_rows_kernel_past_2gib_of_x(ops):
-    """E > 64 with x past 2 GiB (T = 2^19 + 80, H = 2048): the rows kernel addresses each workgroup's own x rows,
+def test_routing_direct_kernel_past_2gib_of_x(ops):
+    """E > 64 with x past 2 GiB (T = 2^19 + 80, H = 2048): the direct kernel addresses each workgroup's own x rows,
     so it still runs and a token's ids and weights are the same bits as when its workgroup's tokens are routed
     alone. The first and the last (partial) token blocks are also checked against the oracle."""
     T, H, E, K = (1 << 19) + 80, 2048, 128, 8
     assert T * H * 2 >= 1 << 31
-    log(f"[rows past 2 GiB] T={T} H={H} E={E} K={K}")
+    log(f"[x past 2 GiB] T={T} H={H} E={E} K={K}")
     x = torch.empty((T, H), dtype=torch.float16, device="cuda")
     ops.synth_normal_f16_(x, 17, synth.STREAM_X, 1.0)
     rng = np.random.default_rng(17)
@@ -394,7 +393,7 @@ def test_routing_rows_kernel_past_2gib_of_x(ops):
         ids_few, w_few = ops.MoeRoutingTopK(x[lo:hi].contiguous(), wg_d, K)
         assert np.array_equal(ids_all[lo:hi], host(ids_few))
         assert np.array_equal(w_all[lo:hi].view(np.uint16), host(w_few).view(np.uint16))
-        check_routing(ids_all[lo:hi], w_all[lo:hi], host(x[lo:hi]), wg, K, f"rows past 2 GiB tokens {lo}-{hi}")
+        check_routing(ids_all[lo:hi], w_all[lo:hi], host(x[lo:hi]), wg, K, f"x past 2 GiB tokens {lo}-{hi}")
     del x
     torch.cuda.empty_cache()
 
@@ -404,17 +403,17 @@ def test_routing_rows_kernel_past_2gib_of_x(ops):
                                      # 55 MB of x (non-temporal x loads), H / 32 = 33 k-steps: a ragged last pair
                                      (26000, 1056, 16, 2)])
 def test_routing_lds_weight_paths(ops, T, H, E, K):
-    """w_gate through LDS: the narrow kernel's transposing-read path (E <= 64) and the rows kernel (E > 64, each
-    wave 16 tokens over all of H). ids and weights against the oracle on every token; for E <= 64 also bit for bit
+    """w_gate rows loaded 16 bytes at a time: the narrow kernel's transposing LDS reads (E <= 64) and the direct kernel
+    (E > 64, transposed in registers). ids and weights against the oracle on every token; for E <= 64 also bit for bit
     against the 2-byte gathers, which run when w_gate is not 16-byte aligned (the same values one fp16 further
-    into a larger buffer)."""
+    into a larger buffer; test_routing_direct_kernel does this for E > 64)."""
     log(f"[lds w_gate] T={T} H={H} E={E} K={K}")
     rng = np.random.default_rng(T + E)
     x = rng.standard_normal((T, H)).astype(np.float16)
     wg = (rng.standard_normal((H, E)) / math.sqrt(H)).astype(np.float16)
     ids_d, w_d = ops.MoeRoutingTopK(dev(x), dev(wg), K)
     ids, w = host(ids_d), host(w_d)
-    check_routing(ids, w, x, wg, K, f"rows T{T} H{H} E{E} K{K}")
+    check_routing(ids, w, x, wg, K, f"lds w_gate T{T} H{H} E{E} K{K}")
     if E <= 64:
         buf = torch.empty(H * E + 8, dtype=torch.float16, device="cuda")
         wg_odd = buf[1: 1 + H * E].view(H, E)  # 2-byte aligned only: the narrow kernel's 2-byte gathers
@@ -1270,16 +1269,16 @@ def test_concurrent_threads_and_streams(ops):
     (2100, 128, 20, 3, 128, 1),    # E % 8 != 0: w_gate by 2-byte loads; 32 experts' blocks
     (9000, 128, 64, 6, 128, 1),    # two 16-token blocks per workgroup, 192 slots per count chunk
     (17000, 128, 13, 2, 128, 1),   # four 16-token blocks; E % 4 != 0 pads the counts rows
-    (3000, 128, 130, 4, 128, 1),   # E > 64: the wide routing kernel counts its 64 tokens
+    (3000, 128, 130, 4, 128, 1),   # E > 64, E % 8 != 0: the direct kernel ranks its 16-token blocks
     (300, 128, 48, 40, 128, 1),    # K = 40: a block's 640 slots are ranked in two passes
-    (1000, 128, 100, 64, 128, 1),  # wide kernel, K = 64: 4096 slots per block, two passes
-    (4096, 256, 128, 8, 128, 1),   # E = 128, T <= 8192: the quarters kernel ranks its 16-token blocks
-    (9000, 256, 128, 4, 128, 1),   # E = 128, T > 8192: the rows kernel ranks its 64-token blocks
+    (1000, 128, 100, 64, 128, 1),  # E % 8 != 0, K = 64: 1024 slots per block of 16 tokens, two passes
+    (4096, 256, 128, 8, 128, 1),   # E = 128, T <= 8192: the direct kernel ranks its 16-token blocks
+    (9000, 256, 128, 4, 128, 1),   # E = 128, T > 8192: the direct kernel ranks its 64-token blocks
     (32790, 1024, 64, 6, 128, 1),  # 32 < E <= 64, T >= 32768: the resident kernel ranks each workgroup's run of
                                    # 9 token blocks (144 tokens, 864 slots) in one pass
     (4, 2048, 256, 8, 128, 0),     # T <= 16, E > 64: split routing (32 workgroups of quarter sums, a selection)
     (16, 1024, 128, 8, 256, 0),    # E = 128: 16 workgroups of quarter sums
-    (3, 1536, 160, 6, 128, 0),     # quarters of 12 k-steps (not a multiple of 8): the quarters kernel routes
+    (3, 1536, 160, 6, 128, 0),     # quarters of 12 k-steps (not a multiple of 8): the direct kernel routes
 ])
 def test_fused_layer_matches_oracle_and_operators(ops, T, H, E, K, I, schedule):
     """moe_layer (routing that also ranks its blocks' slots, one scatter launch, the FFN, the combine): ids and
