@@ -10,8 +10,9 @@ Errors raise MoeError with the library's message, before anything is launched.
 
 A call's own host work is kept to a few microseconds: at decode sizes the kernels of an operator take 5-10 us, and
 asking the library for every shape and entering a stream context took longer than that (T = 8, H = 64, E = 4,
-I = 256, the three operators: 60 us of host time, now 25, of which the four launches take ~13). Shapes that fit are worked out here, any other goes to the library's infer
-function, which words the error; the stream context is entered only for a stream that the caller names.
+I = 256, the three operators: 60 us of host time, now 25, of which the four launches take ~13). Shapes that fit are
+worked out here, any other goes to the library's infer function, which words the error; the stream context is entered
+only for a stream that the caller names.
 """
 from __future__ import annotations
 
@@ -23,6 +24,11 @@ import torch
 from . import _lib
 from ._lib import MoeError, check, dims
 
+# The current stream without the Stream object that torch.cuda.current_stream() makes on each call; both are private to
+# torch, so a torch without them takes the public function.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", None)
+
 _TORCH_DT = {_lib.DT_FLOAT16: torch.float16, _lib.DT_INT32: torch.int32}
 
 
@@ -30,7 +36,9 @@ def _stream_ptr(stream) -> int:
     """The raw stream a call runs on: `stream`, or the current stream of the current device."""
     if stream is not None:
         return int(stream.cuda_stream)
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if _raw_stream is not None and _device is not None:
+        return _raw_stream(_device())
+    return int(torch.cuda.current_stream().cuda_stream)
 
 
 _CURRENT = contextlib.nullcontext()

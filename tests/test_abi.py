@@ -402,3 +402,18 @@ def test_kept_workspace_covers_the_sizes_it_covered(lib, H, E, K, I, kept, sizes
         T = 100 * E // K  # 100 rows per expert: tiled under every line
         assert call(T, query(T, H, E, K, I) - 1) == ERR_WS
         assert call(T, query(T, H, E, K, I)) == ERR_UNSUP
+
+
+def test_current_stream_without_private_torch_functions(monkeypatch):
+    """ops asks torch for the raw current stream through two private functions, through the public one if they are gone."""
+    import types
+
+    import torch
+
+    ops = package().ops
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=77))
+    for name in ("_raw_stream", "_device"):
+        with monkeypatch.context() as m:
+            m.setattr(ops, name, None)
+            assert ops._stream_ptr(None) == 77
+    assert ops._stream_ptr(types.SimpleNamespace(cuda_stream=78)) == 78
