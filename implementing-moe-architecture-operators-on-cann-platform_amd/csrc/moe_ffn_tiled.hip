@@ -26,15 +26,15 @@
 //                  T = 8192, H = 2048, E = 16, K = 2, I = 8192: gate/up 1024 -> 917 -> 888 us, down 506 -> 440 -> 438
 //                  T = 16384, H = 2048, E = 64, K = 6, I = 1408: gate/up 1093 -> 965 -> 940 us, down 587 -> 515 -> 513
 //                What bounds it now is power: on all-zero inputs the first gate/up takes 700 us (942 us in the old
-//                kernel), on random ones the clock falls to ~1.6 GHz. On zeros, without any copies it would take
-//                ~120 us less (L2 misses: with every copy an L2 hit 613 instead of 728 us), without the epilogue
-//                ~60 us less, without the LDS reads nothing less (timing-only copies of the kernel). Measured and
-//                not kept: 32x32x16 MFMAs (9 % slower), MFMAs that share the weight instead of the activation
-//                fragment (1 % slower), copies issued between the MFMAs of the compute ticks (2-7 % slower, they
-//                leave later), the first k-stage rotated per XCD and other cache policies of the copies (level),
-//                s_setprio around the compute tick (level), skipping the second half's ticks in tiles of at most
-//                128 rows (1-3 % slower: such a tile takes as long, and the workgroups that share its weight tile
-//                drift apart).
+//                kernel), on random ones the clock falls to ~1.6 GHz. Timing-only copies of the forms on the way,
+//                on zeros: with four tick pairs a stage (734 us) 615 without any copies after the first stages, 640
+//                without the epilogue, 733 without the LDS reads; with two pairs but 8-byte hidden stores (728 us)
+//                613 with every copy an L2 hit. Measured and not kept: 32x32x16 MFMAs (9 % slower), MFMAs that share
+//                the weight instead of the activation fragment (1 % slower), copies issued between the MFMAs of the
+//                compute ticks (2-7 % slower, they leave later), the first k-stage rotated per XCD and other cache
+//                policies of the copies (level), s_setprio around the compute tick (level), skipping the second
+//                half's ticks in tiles of at most 128 rows (1-3 % slower: such a tile takes as long, and the
+//                workgroups that share its weight tile drift apart).
 //   persistent   one workgroup per CU walks its tiles back to back and the ring runs on across them: the
 //                copies of a tile's first two stages go out during the previous tile's last two. The tile table
 //                (per-expert tile prefix and row offsets) is built once per workgroup in LDS, so finding a tile
@@ -78,7 +78,9 @@ constexpr int kLdsBytes = kNStage * kStageHalfs * 2;  // the ring; the tile tabl
 constexpr int kEpiStageBytes = kThreads / kWave * 2048;  // down epilogue: 16 rows x 128 B per wave
 // LDS of a launch: the ring, the tile table (tab, offs: 2 (E + 1) ints), three row tables, then (down) the
 // epilogue's staging rows at the next 16-byte boundary
-__host__ __device__ constexpr int tiled_epi_stage_offset(int E) { return (kLdsBytes + 8 * (E + 1) + 3 * kBM * 4 + 15) / 16 * 16; }
+__host__ __device__ constexpr int tiled_epi_stage_offset(int E) {
+    return (kLdsBytes + 8 * (E + 1) + 3 * kBM * 4 + 15) / 16 * 16;
+}
 __host__ __device__ constexpr int tiled_lds_bytes(int E, bool down) {
     return down ? tiled_epi_stage_offset(E) + kEpiStageBytes : kLdsBytes + 8 * (E + 1) + 3 * kBM * 4;
 }
@@ -89,9 +91,16 @@ constexpr int kCopyPolicy = 1;  // cache-policy bits of the stage copies: sc0
 constexpr int kMaxParts = 256;
 constexpr int kFixThreads = 256;
 constexpr int kFixRows = 16;  // tile rows per fix-up workgroup
-// The split pays off only while the leftover round is a large share of the down projection: at DeepSeek-V2-Lite
-// prefill (T = 16384, E = 64, K = 6, 13-14 rounds of 22-stage tiles) the kernel before the ticks took 575 us unsplit
-// against 589 us + a 15 us fix-up split (not timed again since); at 2-2.5 rounds (T = 8192, E = 16; Mixtral T = 4096) the split saves 100-215 us.
+// The split pays off only while the leftover round is a large share of the down projection. The whole FFN, leftover
+// round whole / split (us, one box):
+//   H = 2048, E = 16, K = 2, I = 8192   T = 1000 383 / 389, T = 2048 535 / 540, T = 4096 878 / 845,
+//                                       T = 8192 1470 / 1437, T = 12000 2010 / 1957,
+//                                       T = 16384 (5 rounds by the bound) 2737 / 2705
+//   H = 4096, E = 8, K = 2, I = 14336   T = 4096 2467 / 2382, T = 8192 (5 rounds) 4556 / 4461
+//   H = 2048, E = 64, K = 6, I = 1408   T = 1531 275 / 279, T = 4096 478 / 479, T = 16384 (13-14 rounds) 1457 / 1464
+//   H = 1056, E = 24, K = 3, I = 736    T = 3001 83.1 / 87.6
+// so at few rounds of short tiles the fix-up launch costs 1-5 % more than it saves, and at 5 rounds of 128 or 224
+// stages it would still save 1-2 %.
 constexpr int kSplitMaxRounds = 4;
 
 struct TiledArgs {
@@ -102,11 +111,12 @@ struct TiledArgs {
     uint16_t* out;               // hidden or expert_out
     int T, E, K, H, I;
     int kdim;                    // H or I
-    int ndim;                    // I (gate/up: tile covers 128 i of gate and up) or H (down)
-    int ntiles_n;                // n-tiles per expert
+    // [kMaxParts, kBM, kBN] fp32 partial tiles of the split leftover round. It stands between the ints: next to kdim,
+    // ntiles_n and gather would be one scalar load with it and prefill 0.2-0.3 % slower (other scalar registers).
+    float* partial;
+    int ntiles_n;                // n-tiles per expert: 128 i of gate and up, or 256 columns of H (down)
     int gather;                  // gate/up: activation row r -> x[sorted_slot[r] / K]
     int split;                   // split the leftover tiles of each XCD over k (persistent grid <= kMaxParts)
-    float* partial;              // [kMaxParts, kBM, kBN] fp32 partial tiles of the split leftover round
 };
 
 // Work of one XCD: its tiles [base, base + n) are dealt to its nloc workgroups in R full rounds; the L tiles
@@ -147,8 +157,9 @@ __device__ __forceinline__ float swiglu_fast(float g, float u) {
 // The lane index read afresh. Values derived from lane_id() are loop-invariant, so the compiler computes them
 // once and keeps them live across the main loop, where the accumulators and fragments leave no room for them:
 // they are spilled, and each reload in the tile change or the epilogue waits (vmcnt) for every stage copy in
-// flight. A volatile read cannot be hoisted, so what make_plan and the epilogue derive from it is recomputed there.
-// Used by the down projection.
+// flight. A volatile read cannot be hoisted, so what make_plan, the tile search and the epilogue derive from it is
+// recomputed there. Of the six instantiations only the down projection with both SPLIT and KT still spills (one
+// VGPR, to 8 bytes of scratch).
 __device__ __forceinline__ int lane_fresh() {
     int v;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(v));
@@ -296,8 +307,9 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
             for (int jj = 0; jj < kBM / kWave; ++jj) {
                 const int r = jj * kWave + lane;
                 const int row = T.off + min(T.mt * kBM + r, T.ne - 1);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(srsrc, (__attribute__((address_space(3))) void*)(rowtab + buf * kBM + jj * kWave), 4,
-                                                         row * 4, 0, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    srsrc, (__attribute__((address_space(3))) void*)(rowtab + buf * kBM + jj * kWave), 4, row * 4, 0, 0,
+                    0);
             }
         }
     };
@@ -326,16 +338,19 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
             }
         }
         if (p.gather) {
-            P.ar = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.act), 0, static_cast<int>(act_rows * kbytes), 0x00020000);
+            P.ar = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.act), 0,
+                                                     static_cast<int>(act_rows * kbytes), 0x00020000);
         } else {  // the tile's own rows only: any T*K*I stays within 32-bit offsets
             const int row0 = T.off + T.mt * kBM;
             const int rows = min(kBM, T.ne - T.mt * kBM);
-            P.ar = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.act + static_cast<size_t>(row0) * p.kdim), 0,
-                                                     static_cast<int>(static_cast<uint32_t>(rows) * kbytes), 0x00020000);
+            P.ar = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<uint16_t*>(p.act + static_cast<size_t>(row0) * p.kdim), 0,
+                static_cast<int>(static_cast<uint32_t>(rows) * kbytes), 0x00020000);
         }
         const size_t ebase = static_cast<size_t>(T.e) * 3 * static_cast<size_t>(p.I) * p.H;
-        P.wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.w + ebase), 0,
-                                                 static_cast<int>(3u * static_cast<uint32_t>(p.I) * p.H * 2), 0x00020000);
+        P.wr = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint16_t*>(p.w + ebase), 0,
+            static_cast<int>(3u * static_cast<uint32_t>(p.I) * p.H * 2), 0x00020000);
     };
 
     // copies one half tile of stage kc of plan P into ring slot q % 2. The data is consumed from LDS, so the loads
@@ -346,15 +361,17 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
         uint16_t* s = lds + (q % kNStage) * kStageHalfs + h * kHalfTile;
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(P.ar, (__attribute__((address_space(3))) void*)(s + (wave * 2 + j) * 8 * kPitch), 16,
-                                                     static_cast<int>(P.ao[h * 2 + j]), kc * kBK * 2, 0, kCopyPolicy);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                P.ar, (__attribute__((address_space(3))) void*)(s + (wave * 2 + j) * 8 * kPitch), 16,
+                static_cast<int>(P.ao[h * 2 + j]), kc * kBK * 2, 0, kCopyPolicy);
     };
     auto copyB = [&](int q, int h, int kc, const CopyPlan& P) __attribute__((always_inline)) {
         uint16_t* s = lds + (q % kNStage) * kStageHalfs + (2 + h) * kHalfTile;
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(P.wr, (__attribute__((address_space(3))) void*)(s + (wave * 2 + j) * 8 * kPitch), 16,
-                                                     static_cast<int>(P.bo[j]), kc * kBK * 2 + h * bhalf, 0, kCopyPolicy);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                P.wr, (__attribute__((address_space(3))) void*)(s + (wave * 2 + j) * 8 * kPitch), 16,
+                static_cast<int>(P.bo[j]), kc * kBK * 2 + h * bhalf, 0, kCopyPolicy);
     };
     // Accumulators acc[hA][hB]: 4 x 2 blocks of 16 x 16. Fragments: one activation half (4 blocks, both 32-k steps)
     // and both weight halves (2 blocks each).
@@ -364,7 +381,8 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
     auto rdA = [&](int q, int h) __attribute__((always_inline)) {
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
-            const uint16_t* s = lds + (q % kNStage) * kStageHalfs + h * kHalfTile + (wm * 64 + row16) * kPitch + (((kk * 4 + kg) ^ sw) * 8);
+            const uint16_t* s = lds + (q % kNStage) * kStageHalfs + h * kHalfTile + (wm * 64 + row16) * kPitch +
+                                (((kk * 4 + kg) ^ sw) * 8);
 #pragma unroll
             for (int i = 0; i < 4; ++i) fa[kk][i] = *reinterpret_cast<const f16x8*>(s + i * 16 * kPitch);
         }
@@ -372,7 +390,8 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
     auto rdB = [&](int q, int h, f16x8 (&fb)[2][2]) __attribute__((always_inline)) {
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
-            const uint16_t* s = lds + (q % kNStage) * kStageHalfs + (2 + h) * kHalfTile + (wn * 32 + row16) * kPitch + (((kk * 4 + kg) ^ sw) * 8);
+            const uint16_t* s = lds + (q % kNStage) * kStageHalfs + (2 + h) * kHalfTile + (wn * 32 + row16) * kPitch +
+                                (((kk * 4 + kg) ^ sw) * 8);
 #pragma unroll
             for (int j = 0; j < 2; ++j) fb[kk][j] = *reinterpret_cast<const f16x8*>(s + j * 16 * kPitch);
         }
@@ -396,7 +415,9 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
             for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    c[j >> 1][i][j & 1] = mfma16x16x32(j < 2 ? fb0[kk][j & 1] : fb1[kk][j & 1], fa[kk][i], zero && kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : c[j >> 1][i][j & 1]);
+                    c[j >> 1][i][j & 1] =
+                        mfma16x16x32(j < 2 ? fb0[kk][j & 1] : fb1[kk][j & 1], fa[kk][i],
+                                     zero && kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : c[j >> 1][i][j & 1]);
         };
         mma(0);
         if (!KT || !half) mma(1);
@@ -406,7 +427,8 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
     // second activation half. Each refills what the memory tick before it read last: half1 the second activation
     // half of stage q + 1 (stage kc of plan P), half2 the other three half tiles of stage q + 2 (again kc of P).
     int stores = 0;  // stores of this wave's last epilogue, younger than the copies that stage 0 waits for
-    auto half1 = [&](Acc (&acc)[2], int q, bool first, int kc, const CopyPlan& P, bool half) __attribute__((always_inline)) {
+    auto half1 = [&](Acc (&acc)[2], int q, bool first, int kc, const CopyPlan& P, bool half)
+                     __attribute__((always_inline)) {
         rdA(q, 0);
         rdB(q, 0, fb0);
         rdB(q, 1, fb1);
@@ -414,7 +436,8 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
         tick_m(first ? stores : 0);
         tick_c(acc[0], first, half);
     };
-    auto half2 = [&](Acc (&acc)[2], int q, bool first, int kc, const CopyPlan& P, bool half) __attribute__((always_inline)) {
+    auto half2 = [&](Acc (&acc)[2], int q, bool first, int kc, const CopyPlan& P, bool half)
+                     __attribute__((always_inline)) {
         rdA(q, 1);
         copyA(q, 0, kc, P);
         copyB(q, 0, kc, P);
@@ -429,18 +452,20 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
         const int lane_e = lane_fresh(), row16 = lane_e & 15, kg = lane_e >> 4;
         if (SPLIT && cur.part >= 0) {
             // a piece of a split tile: the raw fp32 sums of its k-range, [activation row][weight row] of the tile
-            float* dst = p.partial + static_cast<size_t>(cur.part) * (kBM * kBN) + (wm * 64 + row16) * kBN + wn * 64 + kg * 4;
+            float* dst =
+                p.partial + static_cast<size_t>(cur.part) * (kBM * kBN) + (wm * 64 + row16) * kBN + wn * 64 + kg * 4;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    *reinterpret_cast<f32x4*>(dst + ((i >> 2) * 128 + (i & 3) * 16) * kBN + j * 16) = acc[i >> 2][j >> 1][i & 3][j & 1];
+                    *reinterpret_cast<f32x4*>(dst + ((i >> 2) * 128 + (i & 3) * 16) * kBN + j * 16) =
+                        acc[i >> 2][j >> 1][i & 3][j & 1];
             }
         } else if (EPI == kSwiGLU) {
             // stored through a buffer that ends with the tile's rows; columns past I go past it too
             const int row0 = cur.mt * kBM;
-            const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(p.out + static_cast<size_t>(cur.off + row0) * p.I, 0,
-                                                                                min(kBM, cur.ne - row0) * p.I * 2, 0x00020000);
+            const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(
+                p.out + static_cast<size_t>(cur.off + row0) * p.I, 0, min(kBM, cur.ne - row0) * p.I * 2, 0x00020000);
             const int col = cur.nt * 128 + wn * 32 + (kg & 1) * 16 + (kg >> 1) * 8;
             const uint32_t at = col < p.I ? static_cast<uint32_t>((wm * 64 + row16) * p.I + col) * 2 : 0x80000000u;
 #pragma unroll
@@ -459,11 +484,13 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
                 // odd rows of 16 lanes of block 0 against even ones of block 1: each lane then holds 8 columns in a row
                 const auto lo = __builtin_amdgcn_permlane16_swap(v[0][0], v[1][0], false, false);
                 const auto hi = __builtin_amdgcn_permlane16_swap(v[0][1], v[1][1], false, false);
-                // The row's offset goes into the vector offset. With a scalar one the compiler leaves no wait state between
-                // a 16-byte buffer store and the next write of its data registers (it counts that case as safe), and
-                // where the next instruction was such a write, lanes 12-15 of each row stored the next value.
+                // The row's offset goes into the vector offset. With a scalar one the compiler leaves no wait state
+                // between a 16-byte buffer store and the next write of its data registers (it counts that case as
+                // safe), and where the next instruction was such a write, lanes 12-15 of each row stored the next
+                // value.
                 const uint32_t row = static_cast<uint32_t>(((i >> 2) * 128 + (i & 3) * 16) * p.I) * 2;
-                __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo[0], hi[0], lo[1], hi[1]}, hr, static_cast<int>(at + row), 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo[0], hi[0], lo[1], hi[1]}, hr,
+                                                       static_cast<int>(at + row), 0, 0);
             }
         } else {
             // Whole-line stores: the wave's 128 x 64 sub-tile leaves as 16 instructions of 8 rows x 128 B. Row
@@ -486,7 +513,8 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const f32x4 v = acc[i >> 2][j >> 1][i & 3][j & 1];
-                    *reinterpret_cast<uint2*>(stg + row16 * 128 + (((2 * j + (kg >> 1)) ^ (row16 & 7)) << 4) + ((kg & 1) << 3)) =
+                    *reinterpret_cast<uint2*>(stg + row16 * 128 + (((2 * j + (kg >> 1)) ^ (row16 & 7)) << 4) +
+                                              ((kg & 1) << 3)) =
                         make_uint2(pack_f16(v[0], v[1]), pack_f16(v[2], v[3]));
                 }
                 // the reads take what other lanes of this wave just wrote (LDS operations of one wave run in order)
@@ -572,10 +600,10 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledArgs p) {
 }
 
 // Down projection: adds the pieces of each split leftover tile in piece order (fixed, so the result does not
-// depend on timing) and scatters the fp16 rows to expert_out. Workgroup (g, rb) takes rows [rb * kFixRows, +kFixRows) of leftover tile
-// j = g / 8 of XCD x = g % 8; piece pc of that tile is in the partial slot of workgroup (j * S + pc) * 8 + x of the
-// tiled launch, whose grid had nloc workgroups per XCD. The tile is found as the tiled kernel finds it, from
-// offsets (each wave scans the experts 64 at a time).
+// depend on timing) and scatters the fp16 rows to expert_out. Workgroup (g, rb) takes rows [rb * kFixRows, +kFixRows)
+// of leftover tile j = g / 8 of XCD x = g % 8; piece pc of that tile is in the partial slot of workgroup
+// (j * S + pc) * 8 + x of the tiled launch, whose grid had nloc workgroups per XCD. The tile is found from offsets
+// (each wave scans the experts 64 at a time).
 __global__ __launch_bounds__(kFixThreads) void ffn_tiled_fixup_kernel(TiledArgs p, int nloc) {
     constexpr int nrb = kBM / kFixRows;
     const int rb = static_cast<int>(blockIdx.x) % nrb, g = static_cast<int>(blockIdx.x) / nrb;
@@ -737,19 +765,19 @@ hipError_t launch_ffn_tiled(const uint16_t* x, const uint16_t* expert_weights, u
     p.act = x;
     p.out = ws.hidden;
     p.kdim = H;
-    p.ndim = I;
     p.ntiles_n = (I + 127) / 128;
     p.gather = 1;
     p.partial = ws.partial;
-    // an odd multiple of 32 along the reduction runs the KT instantiation, which clears the last stage's tail
+    // an odd multiple of 32 along the reduction runs the KT instantiation, which multiplies only the first 32-k step of
+    // the last stage
+    const int ggrid = tiled_gateup_grid(T, E, K, I);
     const hipError_t err = H % kBK != 0
-                               ? launch_tiled<kSwiGLU, false, true>(p, tiled_gateup_grid(T, E, K, I), "moe_ffn_gateup_swiglu", stream)
-                               : launch_tiled<kSwiGLU, false, false>(p, tiled_gateup_grid(T, E, K, I), "moe_ffn_gateup_swiglu", stream);
+                               ? launch_tiled<kSwiGLU, false, true>(p, ggrid, "moe_ffn_gateup_swiglu", stream)
+                               : launch_tiled<kSwiGLU, false, false>(p, ggrid, "moe_ffn_gateup_swiglu", stream);
     if (err != hipSuccess) return err;
     p.act = ws.hidden;
     p.out = expert_out;
     p.kdim = I;
-    p.ndim = H;
     p.ntiles_n = (H + kBN - 1) / kBN;
     p.gather = 0;
     p.split = (allow_split && tiled_down_splits(T, E, K, H, I) && ws.partial != nullptr) ? 1 : 0;

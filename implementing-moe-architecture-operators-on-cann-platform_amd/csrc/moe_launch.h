@@ -77,7 +77,6 @@ FfnSplits workspace_splits(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I
 // The workspace a caller is told to give
 size_t workspace_query(int64_t T, int64_t H, int64_t E, int64_t K, int64_t I, bool layer);
 
-int permute_block_threads();
 int permute_chunks(int S);
 int permute_grid(int S, int E);  // workgroups of launch_permute's first launch
 size_t permute_scratch_bytes(int S, int E);

@@ -15,8 +15,8 @@
 //            a scan over the experts gives offsets[e], a scan over its own chunks each chunk's base, and slot s
 //            of expert e in chunk c goes to sorted_slot[offsets[e] + (e's slots in chunks before c) + rank[s]].
 //            Workgroup 0 writes offsets.
-// Few slots (permute_single) whose ids come from the caller (no routing tail) are sorted by one workgroup in one launch,
-// with counts and ranks in LDS and registers (permute_single_kernel).
+// Few slots (permute_single) whose ids come from the caller (no routing tail) are sorted by one workgroup in one
+// launch, with counts and ranks in LDS and registers (permute_single_kernel).
 // No atomics and no cleared memory, so the result is deterministic and needs no memset before the call.
 // Slots whose id is outside [0, E) belong to no expert; the scatter workgroups write zeros into their expert_out
 // rows, each over its own chunks.
@@ -173,7 +173,8 @@ __global__ __launch_bounds__(kScatterThreads) void permute_scatter_kernel(
 // sums over the waves and over the experts then give every slot its row. The other workgroups write zeros into the
 // expert_out rows of ids outside [0, E). Latency bound: one round trip for the ids, ~25 instructions per 64 slots,
 // three barriers. Two launches -> this (us):
-//   S = 800, E = 8 12.3 -> 5.1; S = 2000, E = 16 12.2 -> 4.9; S = 4096, E = 16 12.0 -> 5.5; S = 4097, E = 40 11.4 -> 6.8
+//   S = 800, E = 8 12.3 -> 5.1; S = 2000, E = 16 12.2 -> 4.9; S = 4096, E = 16 12.0 -> 5.5
+//   S = 4097, E = 40 11.4 -> 6.8
 //   S = 9003, E = 24 11.7 -> 9.5; S = 9186, E = 64 11.4 -> 10.4; S = 12288, E = 16 12.1 -> 10.9, E = 128 11.2 -> 14.5
 // The time grows with the slots times the id bits, so the line lies at 64 K of those (permute_single).
 constexpr int kSingleThreads = 1024;
@@ -277,7 +278,6 @@ int id_bits(int E) {
 bool permute_single(int S, int E) { return S <= kSingleSlots && S * id_bits(E) <= 65536; }
 }  // namespace
 
-int permute_block_threads() { return kThreads; }
 int permute_chunks(int S) { return (S + kChunk - 1) / kChunk; }
 int permute_grid(int S, int E) {
     return permute_single(S, E) ? 1 + (S + kSingleThreads - 1) / kSingleThreads : permute_chunks(S);
@@ -317,9 +317,11 @@ hipError_t launch_permute(const int32_t* ids, int S, int E, int H, FfnWorkspace 
         TraceScope trace("moe_permute", stream);
         const int grid = permute_grid(S, E);
         if (S <= kSingleThreads * 4)
-            permute_single_kernel<4><<<grid, kSingleThreads, 0, stream>>>(ids, S, E, H, ws.offsets, ws.sorted_slot, expert_out);
+            permute_single_kernel<4><<<grid, kSingleThreads, 0, stream>>>(ids, S, E, H, ws.offsets, ws.sorted_slot,
+                                                                          expert_out);
         else
-            permute_single_kernel<kSingleIters><<<grid, kSingleThreads, 0, stream>>>(ids, S, E, H, ws.offsets, ws.sorted_slot, expert_out);
+            permute_single_kernel<kSingleIters><<<grid, kSingleThreads, 0, stream>>>(ids, S, E, H, ws.offsets,
+                                                                                     ws.sorted_slot, expert_out);
         return hipGetLastError();
     }
     const int nchunks = permute_chunks(S);

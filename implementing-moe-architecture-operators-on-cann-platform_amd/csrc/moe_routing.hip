@@ -510,7 +510,8 @@ constexpr int row_stage_ksteps(int eb) { return eb >= 16 ? 1 : 16 / eb; }
 // kernels it replaces copied w_gate through LDS and read it back transposed, with one 16 KB stage in flight per wave
 // (up to 8192 tokens), shared a stage between 4 waves behind a barrier (above), or transposed it with LDS stores
 // (E % 8 != 0, or H / 32 odd at E <= 128). Measured, those -> this one (us):
-//   E = 256, H = 7168, K = 8: T = 1 45 -> 35, T = 64 46 -> 39, T = 4096 56 -> 48, T = 8192 110 -> 60, T = 16384 216 -> 112
+//   E = 256, H = 7168, K = 8: T = 1 45 -> 35, T = 64 46 -> 39, T = 4096 56 -> 48, T = 8192 110 -> 60,
+//                             T = 16384 216 -> 112
 //   E = 256, H = 2048, K = 8: T = 64 27 -> 19, T = 4096 30 -> 20, T = 8192 57 -> 28, T = 16384 76 -> 52
 //   E = 128, H = 4096, K = 8: T = 64 21 -> 19, T = 4096 24 -> 20, T = 16384 67 -> 46
 //   E = 80, H = 4640, K = 2, T = 2814 164 -> 20; E = 250, H = 2048, K = 8, T = 16384 172 -> 59;
@@ -551,7 +552,8 @@ __global__ __launch_bounds__(kDirectWaves * kWave, 1) void routing_direct_kernel
     const int t0 = static_cast<int>(blockIdx.x) * (16 * TB);
     const int nks = H / 32, nst = nks / row_stage_ksteps(EB);
     const int kb = row_stage_ksteps(EB) * quarter_begin(wave, nst);
-    const int n = (wave == 3 ? nks : row_stage_ksteps(EB) * quarter_begin(wave + 1, nst)) - kb;  // k-steps of the quarter
+    // k-steps of the quarter
+    const int n = (wave == 3 ? nks : row_stage_ksteps(EB) * quarter_begin(wave + 1, nst)) - kb;
 
     const int rows = min(16 * TB, T - t0);
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
@@ -585,7 +587,8 @@ __global__ __launch_bounds__(kDirectWaves * kWave, 1) void routing_direct_kernel
         auto load_x = [&](f16x8 (&r)[TB], int k) __attribute__((always_inline)) {
 #pragma unroll
             for (int tb = 0; tb < TB; ++tb)
-                r[tb] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(xrs, xo[tb], (kb + min(k, n - 1)) * 64, 0));
+                r[tb] = __builtin_bit_cast(
+                    f16x8, __builtin_amdgcn_raw_buffer_load_b128(xrs, xo[tb], (kb + min(k, n - 1)) * 64, 0));
         };
         f32x4 acc[TB][SP * 8];
 #pragma unroll
@@ -601,11 +604,13 @@ __global__ __launch_bounds__(kDirectWaves * kWave, 1) void routing_direct_kernel
                     u32x4 f;  // expert 8 n + j of the set, rows 8 kg .. 8 kg + 7
 #pragma unroll
                     for (int p = 0; p < 4; ++p)
-                        f[p] = __builtin_amdgcn_perm(r[2 * p + 1][j >> 1], r[2 * p][j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
+                        f[p] = __builtin_amdgcn_perm(r[2 * p + 1][j >> 1], r[2 * p][j >> 1],
+                                                     (j & 1) ? 0x07060302u : 0x05040100u);
 #pragma unroll
                     for (int tb = 0; tb < TB; ++tb)
                         acc[tb][s * 8 + j] = mfma16x16x32(xr[g][tb], __builtin_bit_cast(f16x8, f), acc[tb][s * 8 + j]);
-                    if (j % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // else the fragments of a whole k-step are built at once
+                    // else the fragments of a whole k-step are built at once
+                    if (j % 2 == 1) __builtin_amdgcn_sched_barrier(0);
                 }
             }
         };
@@ -643,7 +648,8 @@ __global__ __launch_bounds__(kDirectWaves * kWave, 1) void routing_direct_kernel
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < TB; ++i) {
-                const int at = wave * TB + i, tb = at / kDirectPhase, b = set0 * 8 + ph * kDirectPhase + at % kDirectPhase;
+                const int at = wave * TB + i, tb = at / kDirectPhase;
+                const int b = set0 * 8 + ph * kDirectPhase + at % kDirectPhase;
                 f32x4 v = part[at * kWave + lane];
 #pragma unroll
                 for (int q = 1; q < kDirectWaves; ++q) v = v + part[(q * TB * kDirectPhase + at) * kWave + lane];
@@ -711,7 +717,8 @@ __global__ __launch_bounds__(kWave) void routing_split_partial_kernel(const uint
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w_gate), 0, H * E * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, T * H * 2, 0x00020000);
     const int xoff = (min(lane / 4, T - 1) * H + (lane % 4) * 8) * 2;
-    // w_gate copy: the narrow kernel's stage layout (wstage_chunk) for GB blocks, columns e0 .. e0 + Gpad - 1 of each row
+    // w_gate copy: the narrow kernel's stage layout (wstage_chunk) for GB blocks, columns e0 .. e0 + Gpad - 1 of each
+    // row
     int woff[16];
 #pragma unroll
     for (int m = 0; m < 16; ++m) {
@@ -1133,11 +1140,15 @@ hipError_t launch_direct(const uint16_t* x, const uint16_t* w_gate, int32_t* ids
 
 // Which kernel routes: the narrow kernel for E <= 64 (or the resident kernel, same bits), the direct kernel above.
 enum RoutingKernel { kNarrowKernel, kResidentKernel, kDirectKernel };
-// Token blocks of 16 per workgroup of the direct kernel, see there: 1 while that makes one round of the CUs (256), then
-// as many as keep w_gate's reads per CU down.
+// Token blocks of 16 per workgroup of the direct kernel, see there. E > 128: 1 while that makes one round of the CUs
+// (256 workgroups), then as many as keep w_gate's reads per CU down. E <= 128 has no 32-token form: from 4097 to 8192
+// tokens 257 to 512 workgroups run in two rounds, each reading all of w_gate (H = 2048, E = 128, K = 8: T = 4096
+// 11.9 us, T = 4200 22.0, T = 8192 23.0, T = 8300 in 64-token blocks 28.0).
 int direct_token_blocks(int T, int eb) { return T > 8192 ? 4 : (T > 4096 && eb == 16 ? 2 : 1); }
-// The LDS a launch reserves: the exchange of the sums and the logits fit in it; a CU holds one workgroup (its waves
-// use most of the register file) whatever it is.
+// The LDS a launch reserves. direct_lds_needed is enough for the exchange of the sums and the logits (24.3 KB at E <= 128
+// and 16 tokens); the sizes here are larger, and part of the plan callers can read. Every form but that one holds one
+// workgroup per CU by its registers alone (277 and more a lane); the one for E <= 128 and 16 tokens (224 registers, two
+// waves per SIMD) is kept to one only by this reservation. Two per CU were not measured.
 size_t direct_lds_bytes(int eb, int tb, bool lw) {
     if (tb < 4) return 4 * (2 * size_t(16384) + 2 * size_t(row_stage_ksteps(eb)) * 1024);
     if (lw) return 4 * size_t(16384) + 4 * (16 + size_t(row_stage_ksteps(eb))) * 1024;
