@@ -49,6 +49,11 @@ def _on(stream):
     return _CURRENT if stream is None else torch.cuda.stream(stream)
 
 
+def _like(t: torch.Tensor) -> torch.Tensor:
+    """What outputs are allocated from: `t` without its class, since new_empty of a tensor subclass gives the subclass."""
+    return t if type(t) is torch.Tensor or type(t) is torch.nn.Parameter else t.as_subclass(torch.Tensor)
+
+
 def _need(t: torch.Tensor, name: str, dtype: torch.dtype) -> None:
     if isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == dtype and t.is_contiguous():
         return
@@ -135,9 +140,10 @@ def MoeRoutingTopK(x: torch.Tensor, w_gate: torch.Tensor, topK: int = 2, stream=
     _need(w_gate, "w_gate", torch.float16)
     T, K = shape = _routing_shape(x, w_gate, topK)
     H, E = w_gate.shape
+    like = _like(x)
     with _on(stream):
-        ids = x.new_empty(shape, dtype=torch.int32)
-        w = x.new_empty(shape)
+        ids = like.new_empty(shape, dtype=torch.int32)
+        w = like.new_empty(shape)
     check(_lib.load().moe_routing_topk(x.data_ptr(), w_gate.data_ptr(), ids.data_ptr(), w.data_ptr(), T, H, E, K,
                                        _stream_ptr(stream)))
     return ids, w
@@ -154,11 +160,12 @@ def MoeExpertFFN(x: torch.Tensor, expert_ids: torch.Tensor, weights: torch.Tenso
     T, H = x.shape
     E, K = expert_weights.shape[0], expert_ids.shape[1]
     lib = _lib.load()
+    like = _like(x)
     with _on(stream):
         if workspace is None:
             need = int(lib.moe_expert_ffn_workspace_bytes(T, H, E, K, inter))
-            workspace = x.new_empty(max(need, 1), dtype=torch.uint8)
-        expert_out = x.new_empty((T, K, H))
+            workspace = like.new_empty(max(need, 1), dtype=torch.uint8)
+        expert_out = like.new_empty((T, K, H))
     check(lib.moe_expert_ffn(x.data_ptr(), expert_ids.data_ptr(), weights.data_ptr(), expert_weights.data_ptr(),
                              expert_out.data_ptr(), workspace.data_ptr(), _bytes(workspace), T, H, E, K, inter,
                              _stream_ptr(stream)))
@@ -180,8 +187,9 @@ def MoeCombine(expert_out: torch.Tensor, expert_ids: torch.Tensor | None, weight
     T, K, H = es
     if weights.shape != es[:2]:
         raise MoeError(3, f"weights shape {tuple(weights.shape)} != {(T, K)}")
+    like = _like(expert_out)
     with _on(stream):
-        y = expert_out.new_empty((T, H))
+        y = like.new_empty((T, H))
     check(_lib.load().moe_combine(expert_out.data_ptr(), _ptr(expert_ids), weights.data_ptr(), y.data_ptr(), T, H, K,
                                   _stream_ptr(stream)))
     return y
@@ -202,12 +210,13 @@ def MoeExpertFFNCombine(x: torch.Tensor, expert_ids: torch.Tensor, weights: torc
     if weights.shape != expert_ids.shape:
         raise MoeError(3, f"weights shape {tuple(weights.shape)} != {(T, K)}")
     lib = _lib.load()
+    like = _like(x)
     with _on(stream):
         if workspace is None:
             need = int(lib.moe_expert_ffn_workspace_bytes(T, H, E, K, inter))
-            workspace = x.new_empty(max(need, 1), dtype=torch.uint8)
-        expert_out = x.new_empty((T, K, H))
-        y = x.new_empty((T, H))
+            workspace = like.new_empty(max(need, 1), dtype=torch.uint8)
+        expert_out = like.new_empty((T, K, H))
+        y = like.new_empty((T, H))
     check(lib.moe_expert_ffn_combine(x.data_ptr(), expert_ids.data_ptr(), weights.data_ptr(),
                                      expert_weights.data_ptr(), expert_out.data_ptr(), y.data_ptr(),
                                      workspace.data_ptr(), _bytes(workspace), T, H, E, K, inter,
@@ -238,14 +247,15 @@ def moe_layer_fused(x: torch.Tensor, w_gate: torch.Tensor, expert_weights: torch
     if expert_weights.shape[0] != E:  # the library takes one E: it would read w_gate past its end or at another stride
         raise MoeError(3, f"w_gate routes to {E} experts, expert_weights holds {expert_weights.shape[0]}")
     lib = _lib.load()
+    like = _like(x)
     with _on(stream):
         if workspace is None:
             need = int(lib.moe_layer_workspace_bytes(T, H, E, K, inter))
-            workspace = x.new_empty(max(need, 1), dtype=torch.uint8)
-        ids = x.new_empty(shape, dtype=torch.int32)
-        w = x.new_empty(shape)
-        expert_out = x.new_empty((T, K, H))
-        y = x.new_empty((T, H))
+            workspace = like.new_empty(max(need, 1), dtype=torch.uint8)
+        ids = like.new_empty(shape, dtype=torch.int32)
+        w = like.new_empty(shape)
+        expert_out = like.new_empty((T, K, H))
+        y = like.new_empty((T, H))
     check(lib.moe_layer(x.data_ptr(), w_gate.data_ptr(), expert_weights.data_ptr(), ids.data_ptr(), w.data_ptr(),
                         expert_out.data_ptr(), y.data_ptr(), workspace.data_ptr(), _bytes(workspace), T, H, E, K,
                         inter, _stream_ptr(stream)))

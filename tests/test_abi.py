@@ -417,3 +417,33 @@ def test_current_stream_without_private_torch_functions(monkeypatch):
             m.setattr(ops, name, None)
             assert ops._stream_ptr(None) == 77
     assert ops._stream_ptr(types.SimpleNamespace(cuda_stream=78)) == 78
+
+
+def test_tensor_subclass_in_plain_tensors_out(monkeypatch):
+    """The operators return plain tensors whatever the class of their inputs (x.new_empty of a subclass gives the
+    subclass). The library is replaced here, so nothing is launched."""
+    import types
+
+    import torch
+
+    class Tagged(torch.Tensor):
+        pass
+
+    ops = package().ops
+    names = ("moe_routing_topk", "moe_expert_ffn", "moe_combine", "moe_expert_ffn_combine", "moe_layer")
+    stub = types.SimpleNamespace(**{n: lambda *a: MOE_OK for n in names}, moe_layer_workspace_bytes=lambda *a: 64,
+                                 moe_expert_ffn_workspace_bytes=lambda *a: 64)
+    monkeypatch.setattr(ops, "_need", lambda *a: None)
+    monkeypatch.setattr(ops, "_stream_ptr", lambda stream: 0)
+    monkeypatch.setattr(ops._lib, "load", lambda: stub)
+
+    def half(*shape):
+        return torch.zeros(shape, dtype=torch.float16)
+
+    ids = torch.zeros((3, 2), dtype=torch.int32)
+    for wrap in (lambda t: t, lambda t: t.as_subclass(Tagged), lambda t: torch.nn.Parameter(t)):
+        x, wg, ew, w, eo = (wrap(t) for t in (half(3, 64), half(64, 8), half(8, 96, 64), half(3, 2), half(3, 2, 64)))
+        outs = [*ops.MoeRoutingTopK(x, wg, 2), ops.MoeExpertFFN(x, ids, w, ew), ops.MoeCombine(eo, ids, w),
+                *ops.MoeExpertFFNCombine(x, ids, w, ew), *ops.moe_layer(x, wg, ew), *ops.moe_layer_fused(x, wg, ew)]
+        assert [type(t) for t in outs] == [torch.Tensor] * 14
+        assert not any(t.requires_grad for t in outs)
