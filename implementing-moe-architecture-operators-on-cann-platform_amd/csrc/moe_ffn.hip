@@ -273,7 +273,8 @@ hipError_t launch_layer(const uint16_t* x, const uint16_t* w_gate, const uint16_
                 err = launch_routing_topk(x, w_gate, ids, weights, T, H, E, K, stream);
             }
             if (err != hipSuccess) return err;
-            return launch_ffn_combine(x, ids, weights, expert_weights, expert_out, y, ws, T, H, E, K, I, stream, splits);
+            return launch_ffn_combine(x, ids, weights, expert_weights, expert_out, y, ws, T, H, E, K, I, stream,
+                                      splits);
         }
         default: return hipErrorInvalidValue;
     }

@@ -50,7 +50,7 @@ def _on(stream):
 
 
 def _like(t: torch.Tensor) -> torch.Tensor:
-    """What outputs are allocated from: `t` without its class, since new_empty of a tensor subclass gives the subclass."""
+    """What outputs are allocated from: `t` without its class (new_empty of a tensor subclass gives the subclass)."""
     return t if type(t) is torch.Tensor or type(t) is torch.nn.Parameter else t.as_subclass(torch.Tensor)
 
 

@@ -405,7 +405,7 @@ def test_kept_workspace_covers_the_sizes_it_covered(lib, H, E, K, I, kept, sizes
 
 
 def test_current_stream_without_private_torch_functions(monkeypatch):
-    """ops asks torch for the raw current stream through two private functions, through the public one if they are gone."""
+    """ops takes the raw current stream from two private torch functions, from the public one if they are gone."""
     import types
 
     import torch

@@ -1485,8 +1485,9 @@ def test_kept_workspace_streams_where_tiled_does_not_fit(ops):
     assert ffn_schedule(T, H, E, K, I) == 1
     lib = ops._lib.load()
     # the least workspace that passes the size check: the call then fails on x's odd address, nothing is launched
+    odd, ok = 0x10001, 0x10000
     least = next(n for n in range(2 * T * K * I, 1 << 24, 256)
-                 if lib.moe_expert_ffn(0x10001, 0x10000, 0x10000, 0x10000, 0x10000, 0x10000, n, T, H, E, K, I, None) == 6)
+                 if lib.moe_expert_ffn(odd, ok, ok, ok, ok, ok, n, T, H, E, K, I, None) == 6)
     log(f"[kept workspace] streaming need {least} bytes, query {ops.workspace_bytes(T, H, E, K, I)}")
     x = torch.empty((T, H), dtype=torch.float16, device="cuda")
     ops.synth_normal_f16_(x, 23, synth.STREAM_X, 1.0)
